@@ -58,7 +58,7 @@ __global__ __launch_bounds__(128) void k_raycast_wave2(SceneDev sc, rlevox_rayma
                                                        int32_t* __restrict__ clip) {
   __shared__ uint4 rcache[64 * RC / 8];
   __shared__ int sweep[64 + kWalkEndWords];
-  __shared__ float dda[kDdaLds];
+  __shared__ __align__(16) float dda[kDdaLds];
   __shared__ ChunkRing ring;
   extern __shared__ uint32_t lds[];
   if ((int)blockIdx.x >= rm.map_line_count) return;

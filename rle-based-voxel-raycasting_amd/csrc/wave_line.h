@@ -42,6 +42,8 @@
 
 #include "device.h"
 
+#include "dda_terms.h"
+
 namespace rlevox {
 
 __device__ inline float readlane_f(float v, int l) {
@@ -247,10 +249,12 @@ __device__ inline int span_draw(const SpanWindow& w, int s1, int e2, float uzb, 
   return (int)__popcll(w.m);
 }
 
-// Uniform DDA walk state of one line (Cuda_Render.h:270-367).
+// DDA walk state of one line (Cuda_Render.h:270-367); uniform but for s, g.
 struct DdaWalk {
-  float dd0, dd1, i0x, i0y, i1x, i1y;  // next crossing distances / positions
-  float g0x, g0y, g1x, g1y, gd0, gd1;  // their increments
+  // Lane j < 6 holds sequence j, its next term s and its increment g: the
+  // next crossing distances dd0, dd1 (0, 1) and the positions i0x, i0y, i1x,
+  // i1y of the x and z crossings (2-5); 0, 2, 3 belong to the x crossings.
+  float s, g;
   float px, py, dnow;                  // last step taken
   int idx;
   int mip, gridx, gridz, mapswitch, shift;
@@ -270,6 +274,160 @@ struct DdaChunk {
   uint2 ent;
 };
 
+// One chunk of the walk from the closed form of its six sequences (lane j < 6
+// passes sequence j's in q).  The walk's order of x and z steps is the merge
+// of the two distance sequences (ties go to x: the walk takes z only when
+// strictly closer).  Lane t guesses i, the x crossings among its t earlier
+// steps, as floor(e0 + e1*t); its own step then says what lane t+1 must hold.
+// While some lane disagrees with its predecessor all take the predecessor's
+// word: the lanes that agree from lane 0 on are the sequential walk's, and
+// each pass adds at least one, so the loop ends with the walk's order.
+// False (nothing written) when the chunk needs terms beyond those fitted.
+//
+// Bound by its own dependent instructions (about 100 in place of the 64
+// chained additions and LDS stores of dda_chain, which took 3.1 K cycles of
+// a walking wavefront's chunk).  The sequences' constants go through LDS and
+// come back as broadcasts: scalar registers for all 30 of them spilled.
+__device__ inline bool dda_merge(DdaWalk& w, DdaChunk& c, const DdaTerms& q, int L, float e0,
+                                 float e1, float nvx, float nvz, bool xseq, float* dl, int lane) {
+  float4* row = reinterpret_cast<float4*>(dl);  // {s, G, c2, G2} of each sequence
+  float* rowK = dl + 24;
+  if (lane < 6) {
+    row[lane] = make_float4(q.s, q.G, q.c2, q.G2);
+    rowK[lane] = q.K;
+  }
+  wave_sync();
+  auto term = [](float4 v, float K, float k) {
+    const bool hi = k > K;
+    return __builtin_fmaf(k, hi ? v.w : v.y, hi ? v.z : v.x);
+  };
+  const float tf = (float)lane;
+  float fi = fminf(fmaxf(floorf(e0 + e1 * tf), 0.0f), tf);
+  float dn, next;
+  bool z;
+  {
+    const float4 A = row[0], B = row[1];
+    const float KA = rowK[0], KB = rowK[1];
+    for (;;) {
+      const float a = term(A, KA, fi), b = term(B, KB, tf - fi);
+      z = b < a;
+      dn = z ? b : a;
+      next = z ? fi : fi + 1.0f;
+      const float told = __int_as_float(dpp_move<0x138>(0, __float_as_int(next)));  // lane 0: 0
+      if (!(__ballot(told != fi) & (~0ull >> (64 - L)))) break;
+      fi = told;
+    }
+  }
+  const float nx = readlane_f(next, L - 1), nz = (float)L - nx;
+  if (nx > nvx || nz > nvz) return false;
+  const float k = z ? tf - fi : fi;
+  const int sx = z ? 4 : 2;
+  const float x = term(row[sx], rowK[sx], k);
+  const float y = term(row[sx + 1], rowK[sx + 1], k);
+  // a step's cell follows from the position before it: the previous lane's
+  c.dn = dn;
+  c.db = __int_as_float(dpp_move<0x138>(__float_as_int(w.dnow), __float_as_int(dn)));
+  c.pbx = __int_as_float(dpp_move<0x138>(__float_as_int(w.px), __float_as_int(x)));
+  c.pby = __int_as_float(dpp_move<0x138>(__float_as_int(w.py), __float_as_int(y)));
+  c.ib = dpp_move<0x138>(w.idx, z ? 1 : 0);
+  w.dnow = readlane_f(dn, L - 1);
+  w.px = readlane_f(x, L - 1);
+  w.py = readlane_f(y, L - 1);
+  w.idx = readlane_i(z ? 1 : 0, L - 1);
+  w.s = dda_term(q, xseq ? nx : nz);
+  wave_sync();
+  return true;
+}
+
+// One chunk of the walk by its own additions, for chunks whose sequences
+// cross more than one binade (a line's first chunk, mostly) or are not
+// finite (rays along an axis).  Lane j < 6 walks sequence j, storing every
+// term to LDS (one add and one store per term for all six sequences at
+// once); each term is made by the same additions the sequential walk makes
+// (the k-th x-crossing term has seen k additions whatever the
+// interleaving).  Lane k then reads term k and finds its merge rank.
+// Layout: six sequences of 65 terms at a stride of 68 floats (the writers,
+// lanes 0..5, hit different LDS banks), then 64 merge slots.
+__device__ inline void dda_chain(DdaWalk& w, DdaChunk& c, int L, float* dl, int lane) {
+  c.db = c.dn = c.pbx = c.pby = 0;
+  c.ib = 0;
+  constexpr int kSeq = 68;
+  float* sA = dl;
+  float* sB = dl + kSeq;
+  float* sX0 = dl + 2 * kSeq;
+  float* sY0 = dl + 3 * kSeq;
+  float* sX1 = dl + 4 * kSeq;
+  float* sY1 = dl + 5 * kSeq;
+  int* slot = reinterpret_cast<int*>(dl + 6 * kSeq);
+  const float dd0 = readlane_f(w.s, 0), dd1 = readlane_f(w.s, 1);
+  const float gd0 = readlane_f(w.g, 0), gd1 = readlane_f(w.g, 1);
+  if (lane < 6) {
+    float t = w.s;
+    float* dst = dl + lane * kSeq;
+    dst[0] = t;
+#pragma unroll
+    for (int k = 1; k <= 64; k++) {  // term 64 is the state after a full chunk
+      t = t + w.g;
+      dst[k] = t;
+    }
+  }
+  wave_sync();
+  const float ak = sA[lane], bk = sB[lane];
+  // Merge ranks: rx = lane + #{j : sB[j] < ak}, rz = lane + #{j : sA[j] <= bk}.
+  // The sequences grow by about gd per term, so a guess g is off by at most
+  // one in practice; three probes around it settle the rank exactly
+  // (the sequences are sorted), else the lane searches.
+  const float qx = (ak - dd1) * __builtin_amdgcn_rcpf(gd1);
+  const float qz = (bk - dd0) * __builtin_amdgcn_rcpf(gd0);
+  const int gx = (int)fminf(fmaxf(ceilf(qx), 0.0f), 64.0f);
+  const int gz = (int)fminf(fmaxf(ceilf(qz), 0.0f), 64.0f);
+  const float bm = sB[max(gx - 1, 0)], b0 = sB[gx], bp = sB[min(gx + 1, 64)];
+  const float am = sA[max(gz - 1, 0)], a0 = sA[gz], ap = sA[min(gz + 1, 64)];
+  const bool okx = (gx == 0 || bm < ak) && (gx >= 63 || !(bp < ak));
+  const bool okz = (gz == 0 || !(bk < am)) && (gz >= 63 || bk < ap);
+  int cx = gx + ((gx < 64 && b0 < ak) ? 1 : 0);
+  int cz = gz + ((gz < 64 && !(bk < a0)) ? 1 : 0);
+  if (!okx) cx = rank_in<false>(sB, ak, gx);
+  if (!okz) cz = rank_in<true>(sA, bk, gz);
+  const int rx = lane + cx;
+  const int rz = lane + cz;
+  if (rx < L) slot[rx] = lane;
+  if (rz < L) slot[rz] = 64 + lane;
+  const int nx = uni((int)__popcll(__ballot(rx < L)));
+  const int nz = L - nx;
+  // The walk's state after the chunk, read in one round trip: the next
+  // terms (index nx of the x sequences, nz of the z sequences) and the last
+  // step, which is the later of x-term nx-1 and z-term nz-1 (a z-term
+  // follows an equal x-term).
+  const float ns = lane < 6 ? dl[lane * kSeq + (((0x0d >> lane) & 1) ? nx : nz)] : 0.0f;
+  const float lA = sA[max(nx - 1, 0)], lX0 = sX0[max(nx - 1, 0)], lY0 = sY0[max(nx - 1, 0)];
+  const float lB = sB[max(nz - 1, 0)], lX1 = sX1[max(nz - 1, 0)], lY1 = sY1[max(nz - 1, 0)];
+  wave_sync();
+  const int cc = lane < L ? slot[lane] : 0;
+  const int p = (lane < L && lane > 0) ? slot[lane - 1] : 0;
+  if (lane < L) {
+    c.dn = cc < 64 ? sA[cc] : sB[cc - 64];
+    if (lane == 0) {
+      c.db = w.dnow;
+      c.pbx = w.px;
+      c.pby = w.py;
+      c.ib = w.idx;
+    } else {
+      c.db = p < 64 ? sA[p] : sB[p - 64];
+      c.pbx = p < 64 ? sX0[p] : sX1[p - 64];
+      c.pby = p < 64 ? sY0[p] : sY1[p - 64];
+      c.ib = p < 64 ? 0 : 1;
+    }
+  }
+  const bool last_z = nz > 0 && (nx == 0 || !(lB < lA));
+  w.dnow = uni_f(last_z ? lB : lA);
+  w.px = uni_f(last_z ? lX1 : lX0);
+  w.py = uni_f(last_z ? lY1 : lY0);
+  w.idx = last_z ? 1 : 0;
+  w.s = ns;
+  wave_sync();
+}
+
 // Advances the walk by one chunk.  Returns false when the line has reached
 // the far distance.
 __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const SceneDev& sc, int zfar,
@@ -285,12 +443,7 @@ __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const SceneDev& s
       w.slab = sc.mip[w.mip].slabs;
       w.shift = sc.mip[w.mip].shift;
     }
-    w.g0x *= 2;
-    w.g0y *= 2;
-    w.g1x *= 2;
-    w.g1y *= 2;
-    w.gd0 *= 2;
-    w.gd1 *= 2;
+    w.g *= 2;
     w.mapswitch *= 2;
     w.dz *= 2;
     w.dzlog++;
@@ -308,109 +461,35 @@ __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const SceneDev& s
   c.mip = w.mip;
   c.shift = w.shift;
   c.slab = w.slab;
-  c.db = c.dn = c.pbx = c.pby = 0;
-  c.ib = 0;
-  // The six crossing sequences (distances, x and z positions of the x and z
-  // crossings) are independent recurrences s <- s + g.  Lane j < 6 walks
-  // sequence j for 63 additions, storing every term to LDS (one add and one
-  // store per term for all six sequences at once); each term is made by the
-  // same additions the sequential walk makes (the k-th x-crossing term has
-  // seen k additions whatever the interleaving).  Lane k then reads term k.
-  // The walk's order of x and z steps is the merge of the two distance
-  // sequences (ties go to x: the walk takes z only when strictly closer).
-  // Layout: six sequences of 65 terms at a stride of 68 floats (the writers,
-  // lanes 0..5, hit different LDS banks), then 64 merge slots.
-  constexpr int kSeq = 68;
-  float* sA = dl;
-  float* sB = dl + kSeq;
-  float* sX0 = dl + 2 * kSeq;
-  float* sY0 = dl + 3 * kSeq;
-  float* sX1 = dl + 4 * kSeq;
-  float* sY1 = dl + 5 * kSeq;
-  int* slot = reinterpret_cast<int*>(dl + 6 * kSeq);
-  {
-    if (lane < 6) {
-      float t = w.dd0, g = w.gd0;
-      t = lane == 1 ? w.dd1 : t;
-      g = lane == 1 ? w.gd1 : g;
-      t = lane == 2 ? w.i0x : t;
-      g = lane == 2 ? w.g0x : g;
-      t = lane == 3 ? w.i0y : t;
-      g = lane == 3 ? w.g0y : g;
-      t = lane == 4 ? w.i1x : t;
-      g = lane == 4 ? w.g1x : g;
-      t = lane == 5 ? w.i1y : t;
-      g = lane == 5 ? w.g1y : g;
-      float* dst = dl + lane * kSeq;
-      dst[0] = t;
-#pragma unroll
-      for (int k = 1; k <= 64; k++) {  // term 64 is the state after a full chunk
-        t = t + g;
-        dst[k] = t;
-      }
+  // Closed form (dda_terms.h): past a line's first chunk, where every
+  // sequence crosses many binades, nearly every chunk's sequences stay in one
+  // or cross into the next one once.
+  bool ok = false;
+  if (w.dnow > 0.0f) {
+    const float sA = readlane_f(w.s, 0), sB = readlane_f(w.s, 1);
+    const float gA = readlane_f(w.g, 0), gB = readlane_f(w.g, 1);
+    // x crossings among the first t steps: the merge of sA + i*gA and
+    // sB + j*gB, i + j = t, wants A's term i-1 <= B's term j and B's term
+    // j-1 < A's term i, so i = floor((sB - sA + gA + t*gB) / (gA + gB))
+    const float gr = __builtin_amdgcn_rcpf(gA + gB);
+    const float e0 = (sB - sA + gA) * gr, e1 = gB * gr;
+    // terms a chunk of L steps may need of either kind (checked afterwards)
+    const float ex = floorf(fminf(fmaxf(e0 + e1 * (float)L, 0.0f), (float)L));
+    const float nvx = ex + 1.0f, nvz = (float)L - ex + 1.0f;
+    const bool xseq = (0x0d >> lane) & 1;  // lanes 0, 2, 3
+    const float nv = xseq ? nvx : nvz;
+    DdaTerms q;
+    bool fit = dda_fit_one(w.s, w.g, nv, q);
+    if ((__ballot(fit) & 0x3f) != 0x3f) {
+      DdaTerms q2;
+      const bool fit2 = dda_fit_two(w.s, w.g, nv, q2, HwRcp());
+      if (!fit) q = q2;
+      fit = fit || fit2;
     }
-    wave_sync();
-    const float ak = sA[lane], bk = sB[lane];
-    // Merge ranks: rx = lane + #{j : sB[j] < ak}, rz = lane + #{j : sA[j] <= bk}.
-    // The sequences grow by about gd per term, so a guess g is off by at most
-    // one in practice; three probes around it settle the rank exactly
-    // (the sequences are sorted), else the lane searches.
-    const float qx = (ak - w.dd1) * __builtin_amdgcn_rcpf(w.gd1);
-    const float qz = (bk - w.dd0) * __builtin_amdgcn_rcpf(w.gd0);
-    const int gx = (int)fminf(fmaxf(ceilf(qx), 0.0f), 64.0f);
-    const int gz = (int)fminf(fmaxf(ceilf(qz), 0.0f), 64.0f);
-    const float bm = sB[max(gx - 1, 0)], b0 = sB[gx], bp = sB[min(gx + 1, 64)];
-    const float am = sA[max(gz - 1, 0)], a0 = sA[gz], ap = sA[min(gz + 1, 64)];
-    const bool okx = (gx == 0 || bm < ak) && (gx >= 63 || !(bp < ak));
-    const bool okz = (gz == 0 || !(bk < am)) && (gz >= 63 || bk < ap);
-    int cx = gx + ((gx < 64 && b0 < ak) ? 1 : 0);
-    int cz = gz + ((gz < 64 && !(bk < a0)) ? 1 : 0);
-    if (!okx) cx = rank_in<false>(sB, ak, gx);
-    if (!okz) cz = rank_in<true>(sA, bk, gz);
-    const int rx = lane + cx;
-    const int rz = lane + cz;
-    if (rx < L) slot[rx] = lane;
-    if (rz < L) slot[rz] = 64 + lane;
-    const int nx = uni((int)__popcll(__ballot(rx < L)));
-    const int nz = L - nx;
-    // The walk's state after the chunk, read in one round trip: the next
-    // terms (index nx of the x sequences, nz of the z sequences) and the last
-    // step, which is the later of x-term nx-1 and z-term nz-1 (a z-term
-    // follows an equal x-term).
-    const float nA = sA[nx], nX0 = sX0[nx], nY0 = sY0[nx];
-    const float nB = sB[nz], nX1 = sX1[nz], nY1 = sY1[nz];
-    const float lA = sA[max(nx - 1, 0)], lX0 = sX0[max(nx - 1, 0)], lY0 = sY0[max(nx - 1, 0)];
-    const float lB = sB[max(nz - 1, 0)], lX1 = sX1[max(nz - 1, 0)], lY1 = sY1[max(nz - 1, 0)];
-    wave_sync();
-    const int cc = lane < L ? slot[lane] : 0;
-    const int p = (lane < L && lane > 0) ? slot[lane - 1] : 0;
-    if (lane < L) {
-      c.dn = cc < 64 ? sA[cc] : sB[cc - 64];
-      if (lane == 0) {
-        c.db = w.dnow;
-        c.pbx = w.px;
-        c.pby = w.py;
-        c.ib = w.idx;
-      } else {
-        c.db = p < 64 ? sA[p] : sB[p - 64];
-        c.pbx = p < 64 ? sX0[p] : sX1[p - 64];
-        c.pby = p < 64 ? sY0[p] : sY1[p - 64];
-        c.ib = p < 64 ? 0 : 1;
-      }
-    }
-    const bool last_z = nz > 0 && (nx == 0 || !(lB < lA));
-    w.dnow = uni_f(last_z ? lB : lA);
-    w.px = uni_f(last_z ? lX1 : lX0);
-    w.py = uni_f(last_z ? lY1 : lY0);
-    w.idx = last_z ? 1 : 0;
-    w.dd0 = uni_f(nA);
-    w.i0x = uni_f(nX0);
-    w.i0y = uni_f(nY0);
-    w.dd1 = uni_f(nB);
-    w.i1x = uni_f(nX1);
-    w.i1y = uni_f(nY1);
-    wave_sync();
+    ok = (__ballot(fit) & 0x3f) == 0x3f &&
+         dda_merge(w, c, q, L, e0, e1, nvx, nvz, xseq, dl, lane);
   }
+  if (!ok) dda_chain(w, c, L, dl, lane);
   w.z += (float)L * w.dz;
   return true;
 }
@@ -455,10 +534,6 @@ __device__ inline void ring_put_dda(ChunkRing& r, int s, const DdaChunk& c, bool
   }
 }
 
-__device__ inline void ring_put_ent(ChunkRing& r, int s, const DdaChunk& c, int lane) {
-  r.ent[s][lane] = c.ent;  // waits for the gather
-}
-
 __device__ inline void ring_get(const ChunkRing& r, int s, DdaChunk& c, int lane) {
   c.L = uni(r.L[s]);
   c.mip = uni(r.mip[s]);
@@ -487,8 +562,8 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
   static_assert(!(COUNT && TWO), "the counting variant walks with one wavefront");
   const int lane = threadIdx.x & 63;
   const bool producer = TWO && threadIdx.x < 64;  // wavefront 0 of a two-wavefront line
-  const int rs = rm.rs;
-  const float half = (float)(rs / 2);
+  const int rs = uni(rm.rs);
+  const float half = uni_f((float)(rs / 2));
   if (lane == 0 && !producer) {
     clip[0] = 0;
     clip[1] = -1;
@@ -525,16 +600,17 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     const float inv = 1.0f / sqrtf(d);
     dir = dir * inv;
   }
-  const float ray_x = rm.cos_myaw * dir.x + rm.sin_myaw * dir.z;
-  const float ray_z = rm.cos_myaw * dir.z - rm.sin_myaw * dir.x;
+  const float ray_x = uni_f(rm.cos_myaw * dir.x + rm.sin_myaw * dir.z);
+  const float ray_z = uni_f(rm.cos_myaw * dir.z - rm.sin_myaw * dir.x);
   const bool vertical = q < 2;
-  const float sin_x = rm.sin_x, cos_x = rm.cos_x;
+  const float sin_x = uni_f(rm.sin_x), cos_x = uni_f(rm.cos_x);
   bool reverse = false;
   if (vertical && ray_z <= 0) reverse = true;
   if (!vertical && ray_x <= 0 && sin_x > 0) reverse = true;
   if (!vertical && ray_x > 0 && sin_x < 0) reverse = true;
   float hmul = reverse ? -half : half;
   if (vertical) hmul = -hmul;
+  hmul = uni_f(hmul);
   const int p_add = reverse ? 1 : -2;
   int p1x = d_f2i((float)rs * p1.x) + p_add;
   int p1y = d_f2i((float)rs * p1.y) + p_add;
@@ -579,7 +655,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
   if (COUNT) cnt.cleared = (uint64_t)(ymax - ymin + 1);
 
   // ---- DDA setup (Cuda_Render.h:270-304), uniform
-  const float vpx = rm.position[0], vpy = rm.position[1], vpz = rm.position[2];
+  const float vpx = uni_f(rm.position[0]), vpy = uni_f(rm.position[1]), vpz = uni_f(rm.position[2]);
   const float ddx = ray_x * rm.cos_y + ray_z * rm.sin_y;
   const float ddy = ray_x * rm.sin_y - ray_z * rm.cos_y;
   float fix_xf = -1, fix_yf = -1, sign_x = -1, sign_y = -1;
@@ -596,18 +672,19 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     frac_y = 1 - frac_y;
   }
   DdaWalk wk;
-  wk.g0y = ddy / fabsf(ddx);
-  wk.g0x = sign_x;
-  wk.g1x = ddx / fabsf(ddy);
-  wk.g1y = sign_y;
-  wk.i0x = wk.g0x * frac_x;
-  wk.i0y = wk.g0y * frac_x;
-  wk.i1x = wk.g1x * frac_y;
-  wk.i1y = wk.g1y * frac_y;
-  wk.gd0 = sqrtf(wk.g0x * wk.g0x + wk.g0y * wk.g0y);
-  wk.gd1 = sqrtf(wk.g1x * wk.g1x + wk.g1y * wk.g1y);
-  wk.dd0 = sqrtf(wk.i0x * wk.i0x + wk.i0y * wk.i0y);
-  wk.dd1 = sqrtf(wk.i1x * wk.i1x + wk.i1y * wk.i1y);
+  {
+    const float g0y = ddy / fabsf(ddx), g1x = ddx / fabsf(ddy);
+    const float g0x = sign_x, g1y = sign_y;
+    const float i0x = g0x * frac_x, i0y = g0y * frac_x, i1x = g1x * frac_y, i1y = g1y * frac_y;
+    const float gv[6] = {sqrtf(g0x * g0x + g0y * g0y), sqrtf(g1x * g1x + g1y * g1y), g0x, g0y, g1x, g1y};
+    const float sv[6] = {sqrtf(i0x * i0x + i0y * i0y), sqrtf(i1x * i1x + i1y * i1y), i0x, i0y, i1x, i1y};
+    wk.s = wk.g = 0;
+#pragma unroll
+    for (int j = 0; j < 6; j++) {
+      wk.s = lane == j ? sv[j] : wk.s;
+      wk.g = lane == j ? gv[j] : wk.g;
+    }
+  }
   wk.px = wk.py = wk.dnow = 0;
   wk.idx = 0;
   wk.mip = 0;
@@ -622,8 +699,8 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
   wk.z = 0;
   wk.yswitch = vpy;
   const float z_add = sin_x;
-  const float y_add = (vertical ? cos_x : 0.0f) * hmul;
-  const int zfar = rm.far_distance;
+  const float y_add = uni_f((vertical ? cos_x : 0.0f) * hmul);
+  const int zfar = uni(rm.far_distance);
   const float mountain = vpy;
   // the early-end test's constants, in LDS behind the sweep marks
   WalkEnd* wend = reinterpret_cast<WalkEnd*>(sweep_lds + 64);
@@ -638,10 +715,9 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
   // of chunk c+1 runs, and while chunk c is replayed the pointer-map gather
   // of chunk c+1 is in flight.  The walk does
   // not depend on the replay (only the line's end does), so a chunk
-  // computed past the end of the line is simply dropped.
-  // The chunk loop is unrolled twice over two register sets (chunk c in one,
-  // c+1 in the other), so the gathered entries never have to be copied (a
-  // copy would wait for the load).
+  // computed past the end of the line is simply dropped.  The step's code
+  // appears once (unrolled over two register sets it took 40 KB of the 64 KB
+  // instruction cache that two compute units share).
   auto chunk_step = [&](auto produce, const DdaChunk& cur, DdaChunk& nxt, bool& have_next) -> bool {
     if (ymin >= ymax) return false;
     const int L = cur.L, mip = cur.mip, shift = cur.shift;
@@ -1157,13 +1233,19 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     return !done;
   };
   if constexpr (!TWO) {
-    DdaChunk ca, cb;
-    bool ha = dda_next_chunk(wk, ca, sc, zfar, dl, lane), hb = false;
-    if (ha) dda_gather(wk, ca, vpx, vpz, fix_xf, fix_yf, lane);
+    DdaChunk cur, nxt;
+    bool have = dda_next_chunk(wk, cur, sc, zfar, dl, lane);
+    if (have) dda_gather(wk, cur, vpx, vpz, fix_xf, fix_yf, lane);
     const std::true_type yes;
-    for (;;) {
-      if (!ha || !chunk_step(yes, ca, cb, hb)) break;
-      if (!hb || !chunk_step(yes, cb, ca, ha)) break;
+    while (have && chunk_step(yes, cur, nxt, have)) {
+      // the copy waits for the gather, whose entries the next step starts with
+      cur.L = nxt.L;
+      cur.mip = nxt.mip;
+      cur.shift = nxt.shift;
+      cur.slab = nxt.slab;
+      cur.db = nxt.db;
+      cur.dn = nxt.dn;
+      cur.ent = nxt.ent;
     }
   } else {
     // Round i: slot i%3 holds chunk i complete, slot (i+1)%3 chunk i+1's DDA
@@ -1174,36 +1256,26 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     // in this round), so they run the same rounds and the same barriers.
     ChunkRing& r = *ring;
     if (producer) {
-      DdaChunk p0, p1;
-      const bool h0 = dda_next_chunk(wk, p0, sc, zfar, dl, lane);
-      ring_put_dda(r, 0, p0, h0, lane);
-      if (h0) dda_gather(wk, p0, vpx, vpz, fix_xf, fix_yf, lane);
-      const bool h1 = h0 && dda_next_chunk(wk, p1, sc, zfar, dl, lane);
-      ring_put_dda(r, 1, p1, h1, lane);
-      if (h0) ring_put_ent(r, 0, p0, lane);
-      if (h1) dda_gather(wk, p1, vpx, vpz, fix_xf, fix_yf, lane);
-      __syncthreads();
-      // two register sets: `pend` holds the chunk whose gather is in flight
-      auto produce_round = [&](int s, DdaChunk& pend, bool& hpend, DdaChunk& nxt) {
-        const int s1 = s == 2 ? 0 : s + 1, s2 = s1 == 2 ? 0 : s1 + 1;
-        const bool h2 = hpend && dda_next_chunk(wk, nxt, sc, zfar, dl, lane);
-        ring_put_dda(r, s2, nxt, h2, lane);
-        if (hpend) ring_put_ent(r, s1, pend, lane);
-        if (h2) dda_gather(wk, nxt, vpx, vpz, fix_xf, fix_yf, lane);
-        hpend = h2;
-      };
-      bool hp = h1;
-      int s = 0;
-      for (;;) {
-        if (!uni(r.have[s])) break;
-        produce_round(s, p1, hp, p0);
-        __syncthreads();
-        if (uni(r.stop[s])) break;
-        s = s == 2 ? 0 : s + 1;
-        if (!uni(r.have[s])) break;
-        produce_round(s, p0, hp, p1);
-        __syncthreads();
-        if (uni(r.stop[s])) break;
+      // chunk n is walked, then chunk n-1's entries stored and chunk n's
+      // gather issued; the barriers after n = 1, 2, ... end the rounds
+      DdaChunk p;
+      uint2 ent = make_uint2(0u, 0u);  // of the gather in flight
+      bool pend = false, more = true;
+      int s = 0, s1 = 2, s2 = 1;  // slots of chunks n, n-1, n-2
+      for (int n = 0;; n++) {
+        if (n >= 2 && !uni(r.have[s2])) break;
+        more = more && dda_next_chunk(wk, p, sc, zfar, dl, lane);
+        ring_put_dda(r, s, p, more, lane);
+        if (pend) r.ent[s1][lane] = ent;  // waits for the gather
+        if (more) {
+          dda_gather(wk, p, vpx, vpz, fix_xf, fix_yf, lane);
+          ent = p.ent;
+        }
+        pend = more;
+        if (n >= 1) __syncthreads();
+        if (n >= 2 && uni(r.stop[s2])) break;
+        s2 = s1;
+        s1 = s;
         s = s == 2 ? 0 : s + 1;
       }
     } else {

@@ -1,0 +1,99 @@
+// The closed form of the DDA's sequences (csrc/dda_terms.h) against the
+// additions it stands for: whenever a fit is accepted for terms 0..n, every
+// one of them equals the sequential fp32 sum bit for bit.  Sums and steps
+// come from seeded lines (all six sequences, doubled at mip switches), plus
+// steps built to tie, to sit at powers of two, at zero, and of any sign.
+// Built and run by tests/test_native_checks.py.
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <random>
+
+#define RLEVOX_HD
+#include "../../rle-based-voxel-raycasting_amd/csrc/dda_terms.h"
+
+using namespace rlevox;
+
+// Nonzero only in the planted build: accepts a first step that differs from
+// the later ones, as a tie leaves it.
+#ifndef DDA_TERMS_PLANT
+#define DDA_TERMS_PLANT 0
+#endif
+
+struct Rcp {
+  float ulps;
+  float operator()(float x) const { return (1.0f / x) * (1.0f + ulps * 1.2e-7f); }
+};
+
+static long tried = 0, one = 0, two = 0, bad = 0;
+
+static void check(float s, float g, int n, float ulps) {
+  DdaTerms q;
+  tried++;
+  bool ok = dda_fit_one(s, g, (float)n, q);
+  if (DDA_TERMS_PLANT && !ok)
+    ok = dda_same_binade(s, fmaf((float)n, q.G, s));
+  if (ok) one++;
+  else if (dda_fit_two(s, g, (float)n, q, Rcp{ulps})) {
+    ok = true;
+    two++;
+  }
+  if (!ok) return;
+  float t = s;
+  for (int k = 0; k <= n; k++) {
+    const float v = dda_term(q, (float)k);
+    if (dda_bits(v) != dda_bits(t)) {
+      if (bad++ < 5) std::printf("s %a g %a n %d term %d: %a, sum %a\n", s, g, n, k, v, t);
+      return;
+    }
+    t = t + g;
+  }
+}
+
+int main() {
+  std::mt19937_64 rng(11);
+  std::uniform_real_distribution<double> U(0.0, 1.0);
+  auto len = [&] { return 1 + (int)(U(rng) * 64); };
+  auto ulps = [&] { return (float)((int)(U(rng) * 5) - 2); };
+  for (int ln = 0; ln < 20000; ln++) {  // the six sequences of a line, chunk by chunk
+    const double ang = U(rng) * 6.283185307179586;
+    const float dx = (float)std::cos(ang), dy = (float)std::sin(ang);
+    const float fx = (float)(U(rng) * 2.0 - 1.0), fy = (float)U(rng);
+    const float sx = dx >= 0 ? 1.0f : -1.0f, sy = dy >= 0 ? 1.0f : -1.0f;
+    float g[6], s[6];
+    g[2] = sx, g[3] = dy / std::fabs(dx), g[4] = dx / std::fabs(dy), g[5] = sy;
+    s[2] = g[2] * fx, s[3] = g[3] * fx, s[4] = g[4] * fy, s[5] = g[5] * fy;
+    g[0] = std::sqrt(g[2] * g[2] + g[3] * g[3]), g[1] = std::sqrt(g[4] * g[4] + g[5] * g[5]);
+    s[0] = std::sqrt(s[2] * s[2] + s[3] * s[3]), s[1] = std::sqrt(s[4] * s[4] + s[5] * s[5]);
+    for (int c = 0; c < 60; c++) {
+      const int n = len();
+      for (int j = 0; j < 6; j++) {
+        check(s[j], g[j], n, ulps());
+        for (int k = 0; k < n; k++) s[j] += g[j];
+        if (c % 16 == 15) g[j] *= 2;
+      }
+    }
+  }
+  for (int i = 0; i < 2000000; i++) {  // arbitrary sums and steps, ties and edges among them
+    float s = std::ldexp((float)U(rng) + 1.0f, (int)(U(rng) * 40) - 20);
+    float g = std::ldexp((float)U(rng) + 1.0f, (int)(U(rng) * 30) - 24);
+    const uint32_t ulp_e = (dda_bits(s) >> 23) - 127 - 23;
+    const int kind = (int)(U(rng) * 8);
+    if (kind == 1) g = std::ldexp((float)((int)(U(rng) * 100000)) + 0.5f, (int)ulp_e);  // ties
+    if (kind == 2) s = std::ldexp(1.0f, (int)(U(rng) * 30) - 10);                        // a power of two
+    if (kind == 3) s = std::nextafterf(std::ldexp(1.0f, (int)(U(rng) * 30) - 10), 0.0f);
+    if (kind == 4) s = 0.0f;
+    if (kind == 5) g = 0.0f;
+    if (kind == 6) g = -g;
+    if (U(rng) < 0.3) s = -s, g = -g;
+    if (i % 1000 == 1) g = INFINITY;
+    if (i % 1000 == 2) s = INFINITY;
+    if (i % 1000 == 3) s = NAN;
+    if (i % 1000 == 4) s = 3.0e38f, g = 1.0e37f;
+    if (i % 1000 == 5) s = std::ldexp(s, -130), g = std::ldexp(g, -130);
+    check(s, g, len(), ulps());
+  }
+  std::printf("dda_terms tried %ld, one binade %ld, one crossing %ld, mismatches %ld\n", tried, one,
+              two, bad);
+  return bad ? 1 : 0;
+}
