@@ -152,15 +152,22 @@ rlevox_status rlevox_scene_upload(rlevox_ctx* ctx, const rlevox_mip* mips, int32
   }
   // Device copy of the descriptor; behind it, scratch for the highest run
   // top of each level (the early end of a line's walk needs the top of the
-  // levels still to come).
+  // levels still to come) and the tops of each level's blocks of columns
+  // (the stretches of a walk that cannot draw).
   void* dd = nullptr;
-  hipError_t e = dev_malloc(&dd, sizeof(SceneDev) + sizeof(int32_t) * RLEVOX_MAX_MIPS);
+  size_t nblocks = 0;
+  for (int i = 0; i < nmips; i++) nblocks += (size_t)skip_blocks(m[i].sx) * skip_blocks(m[i].sz);
+  hipError_t e = dev_malloc(&dd, sizeof(SceneDev) + sizeof(int32_t) * (RLEVOX_MAX_MIPS + nblocks));
   if (e == hipSuccess) {
     s->allocs.push_back(dd);
     int32_t* d_top = (int32_t*)((char*)dd + sizeof(SceneDev));
+    int32_t* d_blocks = d_top + RLEVOX_MAX_MIPS;
     e = launch_fill_u32((uint32_t*)d_top, (uint32_t)INT32_MAX, RLEVOX_MAX_MIPS, nullptr);
-    for (int i = 0; i < nmips && e == hipSuccess; i++)
-      e = launch_column_tops(s->dev.mip[i], i, d_top + i, nullptr);
+    for (int i = 0; i < nmips && e == hipSuccess; i++) {
+      e = launch_column_tops(s->dev.mip[i], i, m[0].sy, d_blocks, d_top + i, nullptr);
+      s->dev.mip[i].tops = d_blocks;
+      d_blocks += (size_t)skip_blocks(m[i].sx) * skip_blocks(m[i].sz);
+    }
     int32_t top[RLEVOX_MAX_MIPS];
     if (e == hipSuccess) e = hipMemcpy(top, d_top, sizeof(top), hipMemcpyDeviceToHost);
     if (e == hipSuccess) {

@@ -50,11 +50,10 @@ __device__ inline int find_view(const ViewDesc* __restrict__ v, int n, int64_t g
 template <bool PAR, int RC>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_raycast_batch(BatchHeader* __restrict__ h,
                                                       const ViewDesc* __restrict__ views) {
-  static_assert(kDdaLds * 4 <= 64 * RC * 2, "DDA scratch must fit in the run cache");
   __shared__ uint32_t bits[(RLEVOX_MAX_RS + 31) / 32];
   __shared__ uint4 rcache[64 * RC / 8];
-  __shared__ int sweep[64 + kWalkEndWords];
-  float* dda = reinterpret_cast<float*>(rcache);  // see kDdaLds
+  __shared__ int sweep[64 + kLineConstWords];
+  __shared__ __align__(16) float dda[kDdaLds];
   const int lane = threadIdx.x;
   const int64_t total = h->total_lines;
   const int nv = h->nviews;
@@ -70,7 +69,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const int x = vd.rm.map_line_count - 1 - (int)((int64_t)g - vd.line_begin);
     render_line_wave<false, false, PAR, RC>(x, *vd.scene, vd.rm,
                                           vd.raybuf + (size_t)x * (size_t)vd.rm.rs,
-                            vd.clip + 2 * x, bits, dda, reinterpret_cast<uint16_t*>(rcache),
+                            vd.clip + 2 * x, bits, dda, (lds_u16*)rcache,
                             sweep, nullptr);
   }
 }

@@ -36,57 +36,60 @@ RLEVOX_HD inline float dda_float(uint32_t u) {
 // zero, with |b| >= |a|, and both are finite.
 RLEVOX_HD inline bool dda_same_binade(float a, float b) {
   const uint32_t x = dda_bits(a), y = dda_bits(b);
-  return ((x ^ y) >> 23) == 0 && y >= x && ((x >> 23) & 0xffu) != 0xffu;
+  return (((x ^ y) >> 23) == 0) & (y >= x) & (((x >> 23) & 0xffu) != 0xffu);
 }
 
+// A sequence at its next term s: terms 0..rem are s + k*G (rem < 0: none
+// known).
+struct DdaSeq {
+  float s, G, rem;
+};
+
+// Fits the sequence from s by g.  rcp: any reciprocal good to a few ulps
+// (the count it gives is checked).
+template <class Rcp>
+RLEVOX_HD inline DdaSeq dda_fit(float s, float g, Rcp rcp) {
+  const float s1 = s + g, s2 = s1 + g;
+  const float G = s1 - s;
+  // the terms below the next power of two
+  const float lim = dda_float((dda_bits(s) & 0xff800000u) + 0x00800000u);
+  float k = floorf((lim - s) * rcp(G));
+  k = fminf(fmaxf(k, 0.0f), 4194304.0f);
+  if (!dda_same_binade(s, fmaf(k, G, s))) k = fmaxf(k - 1.0f, 0.0f);
+  if (!dda_same_binade(s, fmaf(k, G, s))) k = 0.0f;
+  if (s2 - s1 != G) k = fminf(k, 1.0f);
+  // not finite, or a negative zero (which a product with k loses)
+  if (!dda_same_binade(s, s) | (dda_bits(s) == 0x80000000u)) k = -1.0f;
+  return DdaSeq{s, G, k};
+}
+
+// The terms of a chunk, over at most two binades.
 struct DdaTerms {
   float s, G;    // term k = s + k*G for k <= K
   float c2, G2;  // term k = c2 + k*G2 for k > K
   float K;
+  float last;    // up to this term
 };
 
-// One binade: true when terms 0..n of the sequence from s by g are s + k*G.
-RLEVOX_HD inline bool dda_fit_one(float s, float g, float n, DdaTerms& q) {
-  const float s1 = s + g, s2 = s1 + g;
-  q.s = s;
-  q.G = s2 - s1;
-  q.c2 = s;
-  q.G2 = q.G;
-  q.K = n;
-  return s1 - s == q.G && dda_same_binade(s, fmaf(n, q.G, s));
-}
-
-// At most one crossing into another binade within terms 0..n.  rcp: any
-// reciprocal good to a few ulps (the count it gives is checked).
+// Terms past q.rem: the first by its own addition, the others from a fit of
+// their own.
 template <class Rcp>
-RLEVOX_HD inline bool dda_fit_two(float s, float g, float n, DdaTerms& q, Rcp rcp) {
-  const float s1 = s + g, s2 = s1 + g;
-  const float G = s1 - s;
-  // K: the last term in s's binade, i.e. below the next power of two
-  const float lim = dda_float((dda_bits(s) & 0xff800000u) + 0x00800000u);
-  float K = floorf((lim - s) * rcp(G));
-  K = fminf(fmaxf(K, 0.0f), n);
-  if (!dda_same_binade(s, fmaf(K, G, s))) K -= 1.0f;
-  if (dda_same_binade(s, fmaf(K + 1.0f, G, s))) K += 1.0f;
-  const float sK = fmaf(K, G, s);
-  const bool ok1 = K >= 0.0f && dda_same_binade(s, sK) &&
-                   !dda_same_binade(s, fmaf(K + 1.0f, G, s)) && (K < 2.0f || s2 - s1 == G);
-  // past the crossing: the first term by its own addition, then steps of G2
-  const float t0 = sK + g, t1 = t0 + g, t2 = t1 + g;
-  const float G2 = t2 - t1, m = K + 1.0f;
-  const float c2 = fmaf(-m, G2, t0);
-  const bool ok2 = t1 - t0 == G2 && dda_same_binade(t0, fmaf(n - m, G2, t0)) &&
-                   fmaf(m, G2, c2) == t0;
-  q.s = s;
-  q.G = G;
-  q.c2 = c2;
-  q.G2 = G2;
-  q.K = K;
-  return ok1 && ok2 && K < n;
+RLEVOX_HD inline DdaTerms dda_terms(const DdaSeq& q, float g, Rcp rcp) {
+  const float m = q.rem + 1.0f;
+  const DdaSeq r = dda_fit(fmaf(q.rem, q.G, q.s) + g, g, rcp);
+  const float c2 = fmaf(-m, r.G, r.s);
+  const bool ok = (q.rem >= 0.0f) & (r.rem >= 0.0f) & (fmaf(m, r.G, c2) == r.s);
+  return DdaTerms{q.s, q.G, c2, r.G, q.rem, ok ? m + r.rem : q.rem};
 }
 
 RLEVOX_HD inline float dda_term(const DdaTerms& q, float k) {
   return k <= q.K ? fmaf(k, q.G, q.s) : fmaf(k, q.G2, q.c2);
+}
+
+// The sequence k terms on (k <= t.last).
+RLEVOX_HD inline DdaSeq dda_advance(const DdaTerms& t, float k) {
+  const bool hi = k > t.K;
+  return DdaSeq{dda_term(t, k), hi ? t.G2 : t.G, (hi ? t.last : t.K) - k};
 }
 
 }  // namespace rlevox

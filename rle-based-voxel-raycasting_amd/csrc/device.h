@@ -15,6 +15,7 @@
 
 #define RLEVOX_HD __host__ __device__
 #include "walk_end.h"
+#include "walk_skip.h"
 #include "recip_div.h"
 
 namespace rlevox {
@@ -23,6 +24,7 @@ namespace rlevox {
 struct MipDev {
   const uint2* map;
   const uint16_t* slabs;
+  const int32_t* tops;  // highest run top of each kSkipBlock-sided block of columns
   int32_t sx, sz;
   int32_t shift;  // column word offset = map[c].x << shift
   int32_t top;    // highest run top (smallest world row) of this level and all coarser ones

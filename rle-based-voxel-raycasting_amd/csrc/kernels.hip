@@ -38,26 +38,27 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
                                                      uint32_t* __restrict__ raybuf,
                                                      int32_t* __restrict__ clip,
                                                      unsigned long long* counts) {
-  static_assert(kDdaLds * 4 <= 64 * RC * 2, "DDA scratch must fit in the run cache");
   __shared__ uint4 rcache[64 * RC / 8];
-  __shared__ int sweep[64 + kWalkEndWords];
-  float* dda = reinterpret_cast<float*>(rcache);  // see kDdaLds
+  __shared__ int sweep[64 + kLineConstWords];
+  __shared__ __align__(16) float dda[kDdaLds];
   extern __shared__ uint32_t lds[];
   if ((int)blockIdx.x >= rm.map_line_count) return;
   const int x = rm.map_line_count - 1 - (int)blockIdx.x;  // last line first
   render_line_wave<COUNT, false, true, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
                                            clip + 2 * x, lds, dda,
-                                           reinterpret_cast<uint16_t*>(rcache), sweep, counts);
+                                           (lds_u16*)rcache, sweep, counts);
 }
 
 // Two wavefronts (= one block) per ray line: wavefront 0 walks the DDA and
-// gathers the pointer map, wavefront 1 projects, caches and draws.
+// gathers the pointer map, wavefront 1 projects, caches and draws.  Capped at
+// six wavefronts per SIMD (80 registers; it takes 82 to 84 by itself, which
+// leaves five).
 template <int RC>
-__global__ __launch_bounds__(128) void k_raycast_wave2(SceneDev sc, rlevox_raymap rm,
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(6))) void k_raycast_wave2(SceneDev sc, rlevox_raymap rm,
                                                        uint32_t* __restrict__ raybuf,
                                                        int32_t* __restrict__ clip) {
   __shared__ uint4 rcache[64 * RC / 8];
-  __shared__ int sweep[64 + kWalkEndWords];
+  __shared__ int sweep[64 + kLineConstWords];
   __shared__ __align__(16) float dda[kDdaLds];
   __shared__ ChunkRing ring;
   extern __shared__ uint32_t lds[];
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(128) void k_raycast_wave2(SceneDev sc, rlevox_rayma
   const int x = rm.map_line_count - 1 - (int)blockIdx.x;  // last line first
   render_line_wave<false, true, true, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
                                           clip + 2 * x, lds, dda,
-                                          reinterpret_cast<uint16_t*>(rcache), sweep, nullptr,
+                                          (lds_u16*)rcache, sweep, nullptr,
                                           &ring);
 }
 
@@ -160,15 +161,20 @@ hipError_t launch_raycast_plain(const SceneDev& sc, const rlevox_raymap& rm, uin
 
 // The world row of each column's first drawn run (the element walk of
 // Cuda_Render.h:511-524 up to the first element with drawn voxels), reduced
-// to the minimum over the level.  Columns are validated at upload, so the
-// walk stays inside the slab array.
-__global__ __launch_bounds__(256) void k_column_tops(const uint2* __restrict__ map,
-                                                     const uint16_t* __restrict__ slabs, int shift,
-                                                     int level, uint64_t ncols, int32_t* out) {
+// to the minimum over one block of columns per workgroup and over the level.
+// Columns are validated at upload, so the walk stays inside the slab array.
+constexpr int kTopSide = 1 << kSkipBlockLog;
+__global__ __launch_bounds__(kTopSide * kTopSide) void k_column_tops(
+    const uint2* __restrict__ map, const uint16_t* __restrict__ slabs, int shift, int level, int sx,
+    int sz, int32_t empty, int32_t* __restrict__ tops, int32_t* out) {
+  __shared__ int32_t wave_best[kTopSide * kTopSide / 64];
+  const int nx = skip_blocks(sx);
+  const int bz = (int)blockIdx.x / nx, bx = (int)blockIdx.x - bz * nx;
+  const int x = bx * kTopSide + (threadIdx.x & (kTopSide - 1));
+  const int z = bz * kTopSide + (threadIdx.x >> kSkipBlockLog);
   int best = INT32_MAX;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < ncols; c += stride) {
-    const uint2 e = map[c];
+  if (x < sx && z < sz) {
+    const uint2 e = map[(size_t)z * sx + x];
     const uint32_t n = e.y & 0xffffu;
     const uint16_t* runs = slabs + 2 + ((uint64_t)e.x << shift);
     uint32_t w = e.y >> 16;
@@ -177,22 +183,26 @@ __global__ __launch_bounds__(256) void k_column_tops(const uint2* __restrict__ m
       if (k > 0) w = runs[k];
       y += (int)(w & 1023u) << level;
       if (w >> 10) {
-        best = min(best, y);
+        best = y;
         break;
       }
     }
   }
   for (int o = 32; o > 0; o >>= 1) best = min(best, __shfl_xor(best, o));
-  if ((threadIdx.x & 63) == 0 && best != INT32_MAX) atomicMin(out, best);
+  if ((threadIdx.x & 63) == 0) wave_best[threadIdx.x >> 6] = best;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < kTopSide * kTopSide / 64; i++) best = min(best, wave_best[i]);
+    tops[blockIdx.x] = min(best, empty);
+    if (best != INT32_MAX) atomicMin(out, best);
+  }
 }
 
-hipError_t launch_column_tops(const MipDev& m, int level, int32_t* out, hipStream_t s) {
-  const uint64_t ncols = (uint64_t)m.sx * (uint64_t)m.sz;
-  if (ncols == 0) return hipSuccess;
-  uint64_t blocks = (ncols + 255) / 256;
-  if (blocks > 8192) blocks = 8192;
-  hipLaunchKernelGGL(k_column_tops, dim3((unsigned)blocks), dim3(256), 0, s, m.map, m.slabs,
-                     m.shift, level, ncols, out);
+hipError_t launch_column_tops(const MipDev& m, int level, int32_t empty, int32_t* tops,
+                              int32_t* out, hipStream_t s) {
+  const int64_t blocks = (int64_t)skip_blocks(m.sx) * skip_blocks(m.sz);
+  hipLaunchKernelGGL(k_column_tops, dim3((unsigned)blocks), dim3(kTopSide * kTopSide), 0, s, m.map,
+                     m.slabs, m.shift, level, m.sx, m.sz, empty, tops, out);
   return hipGetLastError();
 }
 

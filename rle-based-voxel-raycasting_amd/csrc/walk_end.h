@@ -31,47 +31,53 @@ namespace rlevox {
 // truncates to <= ymin the walk is over.
 struct WalkEnd {
   static constexpr float kRel = 1e-4f, kAbs = 0.125f;
-  float kz, sx, cx, R, rx, rz, half, m, lim;
-  int on, vertical;
+  // pz = kz*d + sx*y, py = kd*d + ky*y; ad, ay: the magnitudes that go into
+  // py per d and per y; half; m: eye row offset; lim: the horizon limit
+  float kz, sx, kd, ky, ad, ay, half, m, lim;
+  int on;
 
   // The line's constants; cos_x, sin_x: of the pitch; hmul: the signed half
   // render size multiplying py (Cuda_Render.h:208-210); mountain: eye row
   // offset (viewpos.y).
   RLEVOX_HD void init(float cos_x, float sin_x, float hmul, float ray_x, float ray_z, bool vert,
                        float mountain, float half_) {
-    cx = cos_x;
+    kz = cos_x * ray_z;
     sx = sin_x;
-    R = hmul;
-    rx = ray_x;
-    rz = ray_z;
+    kd = vert ? -hmul * sin_x * ray_z : hmul * ray_x;
+    ky = vert ? hmul * cos_x : 0.0f;
+    ad = fabsf(hmul) * (fabsf(sin_x * ray_z) + fabsf(ray_x));
+    ay = fabsf(hmul * cos_x);
     half = half_;
     m = mountain;
-    vertical = vert ? 1 : 0;
-    kz = cos_x * ray_z;
     on = kz > 0.0f ? 1 : 0;  // pz must grow with d (else far cells fall behind the eye)
     lim = 0.0f;
     if (on) {  // the horizon limit d -> inf, with its margin
-      const float pyk = (vert ? -hmul * sin_x * ray_z : hmul * ray_x) / kz;
-      const float pya = fabsf(hmul) * (fabsf(sin_x * ray_z) + fabsf(ray_x)) / kz;
-      lim = half + pyk + kRel * (fabsf(half) + fabsf(pyk) + pya);
+      const float pyk = kd / kz;
+      lim = half + pyk + kRel * (fabsf(half) + fabsf(pyk) + ad / kz);
     }
   }
 
-  // Bound (with margin) at distance d and height y; ok = false when pz is
-  // not safely positive there.
-  RLEVOX_HD float corner(float d, float y, bool& ok) const {
-    const float pz = kz * d + sx * y;
-    const float pza = kz * d + fabsf(sx * y);
-    if (!(pz > 1e-3f * pza) || !(pz > 1e-3f)) {
-      ok = false;
-      return 0.0f;
-    }
-    const float py = vertical ? R * (cx * y - sx * rz * d) : R * rx * d;
-    const float pya = fabsf(R) * (fabsf(cx * y) + fabsf(sx * rz * d) + fabsf(rx * d));
-    // one division: the products' rounding (a few ulps) is far inside the margin
+  // What a bound needs of a distance (>= 0) and of a height.
+  struct D {
+    float z, y, a;
+  };
+  RLEVOX_HD D at_d(float d) const { return D{kz * d, kd * d, ad * d}; }
+  RLEVOX_HD D at_y(float y) const { return D{sx * y, ky * y, ay * fabsf(y)}; }
+
+  // Bound (with margin) at a distance and a height; ok = false when pz is
+  // not safely positive there.  The reciprocal may be off by some ulps (the
+  // hardware's is by one): like the products' rounding that is far inside
+  // the margin.
+  RLEVOX_HD float corner(const D& d, const D& y, bool& ok) const {
+    const float pz = d.z + y.z, pza = fabsf(d.z) + fabsf(y.z);
+    ok = ok & (pz > 1e-3f * pza) & (pz > 1e-3f);
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float inv = __builtin_amdgcn_rcpf(pz);
+#else
     const float inv = 1.0f / pz;
-    const float q = py * inv;
-    return half + q + kRel * (fabsf(half) + fabsf(q) * (pza * inv) + pya * inv);
+#endif
+    const float q = (d.y + y.y) * inv;
+    return half + q + kRel * (fabsf(half) + (fabsf(q) * pza + (d.a + y.a)) * inv);
   }
 
   // A value no bound falls below: while ymin + (1 - kAbs) <= floor_(), done()
@@ -85,10 +91,10 @@ struct WalkEnd {
   RLEVOX_HD bool done(float D0, int ymin, int top, int sy) const {
     if (!on) return false;
     bool ok = true;
-    const float a = corner(D0, m + (float)top, ok);
-    const float b = corner(D0, m + (float)sy, ok);
-    if (!ok) return false;
-    return fmaxf(fmaxf(a, b), lim) < (float)ymin + (1.0f - kAbs);
+    const D d = at_d(D0);
+    const float a = corner(d, at_y(m + (float)top), ok);
+    const float b = corner(d, at_y(m + (float)sy), ok);
+    return ok && fmaxf(fmaxf(a, b), lim) < (float)ymin + (1.0f - kAbs);
   }
 };
 // 32-bit words of a WalkEnd kept in LDS by the wavefront kernels (read once

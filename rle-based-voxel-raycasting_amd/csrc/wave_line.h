@@ -30,8 +30,9 @@
 //     increments k times from the span start, exactly as the pixel loop
 //     does (Cuda_Render.h:687), and the line's LDS bitmap is updated from a
 //     ballot of the drawn pixels.
-//  7. The walk ends once no later step can draw (walk_end.h), leaving the
-//     line as the full walk to the far distance does.
+//  7. The walk ends once no later step can draw (walk_end.h), and steps over
+//     stretches that cannot (walk_skip.h), leaving the line as the full walk
+//     to the far distance does.
 //  8. Two-wavefront form (k_raycast_wave2): one wavefront walks the DDA and
 //     gathers (1-2), the other projects, caches and draws (3-7); chunks pass
 //     between them through a three-slot LDS ring with one workgroup barrier
@@ -82,11 +83,26 @@ __device__ inline void wave_sync() {
 // The default depth; the wavefront-per-line kernels are also built for 24
 // and 56 words (a tuning choice).
 constexpr int kRunCache = 40;
-// LDS floats per wavefront used by the DDA chunk.  The kernels place them in
-// the run cache's memory: the DDA of chunk c+1 runs after chunk c's replay
-// has finished with the cache and before chunk c+1's cache is stored.
+// The cache holds 16-byte words of 8 slab words, word i of all 64 lanes'
+// columns side by side: the layout in which the loads write LDS themselves
+// (global_load_lds_dwordx4: lane l's 16 bytes go to the base + 16*l), so no
+// register holds them on the way.  20 to 28 registers did, across the next
+// chunk's DDA, and the batch kernel spilled.
+// Slab word j (from the 16-byte boundary) of a lane's column:
+__device__ inline int rc_index(int lane, int j) { return ((j & ~7) << 6) + (lane << 3) + (j & 7); }
+
+// The cache as LDS (the loads into it need the address space).
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+
+// One column of the cache: word i from the column header on.
+struct RcColumn {
+  const lds_u16* rc;
+  int lane, delta;
+  __device__ uint16_t operator[](int i) const { return rc[rc_index(lane, delta + i)]; }
+};
+
+// LDS floats per wavefront used by the DDA chunk.
 constexpr int kDdaLds = 6 * 68 + 64;
-static_assert(kDdaLds * 4 <= 64 * kRunCache * 2, "DDA scratch must fit in the run cache");
 
 // First y in [from, to) whose bit is clear, or `to` (from <= to).
 __device__ inline int first_clear(const uint32_t* bits, int from, int to, int lane) {
@@ -165,7 +181,7 @@ __device__ inline void bits_or(uint32_t* bits, int base, uint64_t m, int lane) {
 // Draws pixels [y0, s2) of one span (uniform arguments; Cuda_Render.h:
 // 678-733).  Pixel y0+k has had k per-pixel increments.
 __device__ inline int draw_span(int y0, int s2, float uzb, float ozb, float u2dz, float onedz2,
-                                float tlo, float thi, const uint16_t* cached, int ccap,
+                                float tlo, float thi, RcColumn cached, int ccap,
                                 const uint16_t* colours, int cofs, uint32_t* __restrict__ row,
                                 uint32_t* bits, int lane) {
   int drawn = 0;
@@ -226,7 +242,7 @@ __device__ inline SpanWindow span_window(const uint32_t* bits, int s1, int e2, i
 // had k per-pixel increments.
 __device__ inline int span_draw(const SpanWindow& w, int s1, int e2, float uzb, float ozb,
                                 float u2dz, float onedz2, float tlo, float thi,
-                                const uint16_t* cached, int ccap, const uint16_t* colours,
+                                RcColumn cached, int ccap, const uint16_t* colours,
                                 int cofs, uint32_t* __restrict__ row, uint32_t* bits, int lane) {
   if (!w.fused)
     return draw_span(w.y0, e2, uzb, ozb, u2dz, onedz2, tlo, thi, cached, ccap, colours, cofs, row,
@@ -251,14 +267,21 @@ __device__ inline int span_draw(const SpanWindow& w, int s1, int e2, float uzb, 
 
 // DDA walk state of one line (Cuda_Render.h:270-367); uniform but for s, g.
 struct DdaWalk {
-  // Lane j < 6 holds sequence j, its next term s and its increment g: the
-  // next crossing distances dd0, dd1 (0, 1) and the positions i0x, i0y, i1x,
-  // i1y of the x and z crossings (2-5); 0, 2, 3 belong to the x crossings.
-  float s, g;
+  // Lane j < 6 holds sequence j, its next term and fit q and its increment g:
+  // the next crossing distances dd0, dd1 (0, 1) and the positions i0x, i0y,
+  // i1x, i1y of the x and z crossings (2-5); 0, 2, 3 belong to the x
+  // crossings.
+  DdaSeq q;
+  float g;
   float px, py, dnow;                  // last step taken
   int idx;
   int mip, gridx, gridz, mapswitch, shift;
   int dzlog;  // dz = 2^dzlog
+  // The window of steps the walk has looked ahead over: lane g holds the
+  // bound of its steps 8g..8g+7 (walk_skip.h); the walk's next step in it
+  // (negative: still before it), its length.
+  float bound;
+  int ofs, end;
   float dz, z, yswitch;
   const uint2* map;
   const uint16_t* slab;
@@ -268,6 +291,7 @@ struct DdaWalk {
 // pointer-map entry.  The mip level is constant within a chunk.
 struct DdaChunk {
   int L, mip, shift;
+  int first;  // lanes below hold no step of the line's own
   const uint16_t* slab;
   float db, dn, pbx, pby;  // per lane: distances and position before the step
   int ib;
@@ -282,14 +306,17 @@ struct DdaChunk {
 // While some lane disagrees with its predecessor all take the predecessor's
 // word: the lanes that agree from lane 0 on are the sequential walk's, and
 // each pass adds at least one, so the loop ends with the walk's order.
-// False (nothing written) when the chunk needs terms beyond those fitted.
+// The chunk may begin T steps on: lane 0 then settles i against the terms
+// before it.  What came before lane 0's step is not made out (c.first = 1):
+// the caller lets the chunk begin one step early, on one that cannot draw.
+// False (the walk unchanged) when the chunk needs terms beyond those fitted.
 //
 // Bound by its own dependent instructions (about 100 in place of the 64
 // chained additions and LDS stores of dda_chain, which took 3.1 K cycles of
 // a walking wavefront's chunk).  The sequences' constants go through LDS and
 // come back as broadcasts: scalar registers for all 30 of them spilled.
-__device__ inline bool dda_merge(DdaWalk& w, DdaChunk& c, const DdaTerms& q, int L, float e0,
-                                 float e1, float nvx, float nvz, bool xseq, float* dl, int lane) {
+__device__ inline bool dda_merge(DdaWalk& w, DdaChunk& c, const DdaTerms& q, int T, int L, float e0,
+                                 float e1, bool xseq, float* dl, int lane) {
   float4* row = reinterpret_cast<float4*>(dl);  // {s, G, c2, G2} of each sequence
   float* rowK = dl + 24;
   if (lane < 6) {
@@ -301,7 +328,7 @@ __device__ inline bool dda_merge(DdaWalk& w, DdaChunk& c, const DdaTerms& q, int
     const bool hi = k > K;
     return __builtin_fmaf(k, hi ? v.w : v.y, hi ? v.z : v.x);
   };
-  const float tf = (float)lane;
+  const float tf = (float)(T + lane);
   float fi = fminf(fmaxf(floorf(e0 + e1 * tf), 0.0f), tf);
   float dn, next;
   bool z;
@@ -313,13 +340,21 @@ __device__ inline bool dda_merge(DdaWalk& w, DdaChunk& c, const DdaTerms& q, int
       z = b < a;
       dn = z ? b : a;
       next = z ? fi : fi + 1.0f;
-      const float told = __int_as_float(dpp_move<0x138>(0, __float_as_int(next)));  // lane 0: 0
+      float own = fi;  // lane 0's: 0 at T = 0
+      if (T > 0) {
+        const bool few = tf > fi && !(term(B, KB, tf - fi - 1.0f) < a);
+        const bool many = fi > 0.0f && b < term(A, KA, fi - 1.0f);
+        own += few ? 1.0f : (many ? -1.0f : 0.0f);
+      }
+      const float told = __int_as_float(dpp_move<0x138>(__float_as_int(own), __float_as_int(next)));
       if (!(__ballot(told != fi) & (~0ull >> (64 - L)))) break;
       fi = told;
     }
   }
-  const float nx = readlane_f(next, L - 1), nz = (float)L - nx;
-  if (nx > nvx || nz > nvz) return false;
+  // the terms after the chunk's last step must still be within the fits
+  const float nx = readlane_f(next, L - 1);
+  const float n = xseq ? nx : (float)(T + L) - nx;
+  if (__ballot(n > q.last) & 0x3f) return false;
   const float k = z ? tf - fi : fi;
   const int sx = z ? 4 : 2;
   const float x = term(row[sx], rowK[sx], k);
@@ -330,11 +365,12 @@ __device__ inline bool dda_merge(DdaWalk& w, DdaChunk& c, const DdaTerms& q, int
   c.pbx = __int_as_float(dpp_move<0x138>(__float_as_int(w.px), __float_as_int(x)));
   c.pby = __int_as_float(dpp_move<0x138>(__float_as_int(w.py), __float_as_int(y)));
   c.ib = dpp_move<0x138>(w.idx, z ? 1 : 0);
+  c.first = T > 0 ? 1 : 0;
   w.dnow = readlane_f(dn, L - 1);
   w.px = readlane_f(x, L - 1);
   w.py = readlane_f(y, L - 1);
   w.idx = readlane_i(z ? 1 : 0, L - 1);
-  w.s = dda_term(q, xseq ? nx : nz);
+  w.q = dda_advance(q, n);
   wave_sync();
   return true;
 }
@@ -351,6 +387,7 @@ __device__ inline bool dda_merge(DdaWalk& w, DdaChunk& c, const DdaTerms& q, int
 __device__ inline void dda_chain(DdaWalk& w, DdaChunk& c, int L, float* dl, int lane) {
   c.db = c.dn = c.pbx = c.pby = 0;
   c.ib = 0;
+  c.first = 0;
   constexpr int kSeq = 68;
   float* sA = dl;
   float* sB = dl + kSeq;
@@ -359,10 +396,10 @@ __device__ inline void dda_chain(DdaWalk& w, DdaChunk& c, int L, float* dl, int 
   float* sX1 = dl + 4 * kSeq;
   float* sY1 = dl + 5 * kSeq;
   int* slot = reinterpret_cast<int*>(dl + 6 * kSeq);
-  const float dd0 = readlane_f(w.s, 0), dd1 = readlane_f(w.s, 1);
+  const float dd0 = readlane_f(w.q.s, 0), dd1 = readlane_f(w.q.s, 1);
   const float gd0 = readlane_f(w.g, 0), gd1 = readlane_f(w.g, 1);
   if (lane < 6) {
-    float t = w.s;
+    float t = w.q.s;
     float* dst = dl + lane * kSeq;
     dst[0] = t;
 #pragma unroll
@@ -424,74 +461,150 @@ __device__ inline void dda_chain(DdaWalk& w, DdaChunk& c, int L, float* dl, int 
   w.px = uni_f(last_z ? lX1 : lX0);
   w.py = uni_f(last_z ? lY1 : lY0);
   w.idx = last_z ? 1 : 0;
-  w.s = ns;
+  w.q.s = ns;
+  w.q.rem = -1.0f;
   wave_sync();
 }
 
-// Advances the walk by one chunk.  Returns false when the line has reached
-// the far distance.
-__device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const SceneDev& sc, int zfar,
-                                      float* dl, int lane) {
-  // distance mip switch (Cuda_Render.h:343-365), uniform
-  while (w.z > (float)w.mapswitch || w.yswitch > 512.0f) {
-    w.yswitch = w.yswitch * 0.5f;
-    if (w.mip < sc.nmips - 1) {
-      w.mip++;
-      w.gridx >>= 1;
-      w.gridz >>= 1;
-      w.map = sc.mip[w.mip].map;
-      w.slab = sc.mip[w.mip].slabs;
-      w.shift = sc.mip[w.mip].shift;
+// What the walk's own constants cost to hold across a line goes to LDS.
+struct LineConsts {
+  WalkEnd end;
+  SkipLine line;
+};
+constexpr int kLineConstWords = (int)(sizeof(LineConsts) / 4);
+
+// The bounds of the window that begins `ahead` steps on, n steps before the
+// next mip switch or the far distance.
+__device__ inline void dda_look_ahead(DdaWalk& w, const SceneDev& sc, const LineConsts& lc,
+                                      int ahead, int n, int lane) {
+  const float sA = readlane_f(w.q.s, 0), sB = readlane_f(w.q.s, 1);
+  const float gA = readlane_f(w.g, 0), gB = readlane_f(w.g, 1);
+  const float r = __builtin_amdgcn_rcpf(gA + gB);
+  const SkipBase b{w.px, w.py, w.dnow, sA, sB, gA, gB, (sB - sA + gA) * r, gB * r};
+  const SkipLevel v{w.mip, w.gridx, w.gridz, sc.mip[w.mip].tops, sc.mip[w.mip].top};
+  const int t0 = ahead + lane * kSkipSteps;
+  const float bound = skip_bound(lc.end, lc.line, b, v, sc.sy, t0, t0 + kSkipSteps);
+  w.bound = t0 < n ? bound : -__builtin_inff();
+  w.ofs = -ahead;
+  w.end = min(kSkipWindow, n - ahead);
+}
+
+// Steps that cannot draw are looked for up to this far ahead (the chunk's
+// steps are counted in floats, and its terms come from two binades).
+constexpr int kSkipReach = 2048;
+
+// Advances the walk by one chunk of up to 64 steps.  SKIP: steps that cannot
+// draw above the horizon row ymin (a row the line has reached or passed) are
+// stepped over on the way.  Returns false when the line has reached the far
+// distance.
+template <bool SKIP>
+__device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const SceneDev& sc,
+                                      const LineConsts& lc, int zfar, int ymin, float* dl,
+                                      int lane) {
+  for (;;) {
+    // distance mip switch (Cuda_Render.h:343-365), uniform
+    while (w.z > (float)w.mapswitch || w.yswitch > 512.0f) {
+      w.yswitch = w.yswitch * 0.5f;
+      if (w.mip < sc.nmips - 1) {
+        w.mip++;
+        w.gridx >>= 1;
+        w.gridz >>= 1;
+        w.map = sc.mip[w.mip].map;
+        w.slab = sc.mip[w.mip].slabs;
+        w.shift = sc.mip[w.mip].shift;
+      }
+      w.g *= 2;
+      w.mapswitch *= 2;
+      w.dz *= 2;
+      w.dzlog++;
+      w.ofs = w.end = 0;
+      w.q.rem = -1.0f;
     }
-    w.g *= 2;
-    w.mapswitch *= 2;
-    w.dz *= 2;
-    w.dzlog++;
-  }
-  // Iterations left before the next mip switch and before z passes z_far.
-  // z, dz = 2^dzlog and mapswitch are exact integers below 2^31, and
-  // z <= mapswitch here; a negative distance to z_far ends the line either
-  // way, so the shifts decide exactly as the divisions would.
-  const int zi = (int)w.z;
-  const int n_mip = ((w.mapswitch - zi) >> w.dzlog) + 1;
-  const int n_far = (zfar - zi) >> w.dzlog;
-  if (n_far <= 0) return false;
-  const int L = min(64, min(n_mip, n_far));
-  c.L = L;
-  c.mip = w.mip;
-  c.shift = w.shift;
-  c.slab = w.slab;
-  // Closed form (dda_terms.h): past a line's first chunk, where every
-  // sequence crosses many binades, nearly every chunk's sequences stay in one
-  // or cross into the next one once.
-  bool ok = false;
-  if (w.dnow > 0.0f) {
-    const float sA = readlane_f(w.s, 0), sB = readlane_f(w.s, 1);
-    const float gA = readlane_f(w.g, 0), gB = readlane_f(w.g, 1);
-    // x crossings among the first t steps: the merge of sA + i*gA and
-    // sB + j*gB, i + j = t, wants A's term i-1 <= B's term j and B's term
-    // j-1 < A's term i, so i = floor((sB - sA + gA + t*gB) / (gA + gB))
-    const float gr = __builtin_amdgcn_rcpf(gA + gB);
-    const float e0 = (sB - sA + gA) * gr, e1 = gB * gr;
-    // terms a chunk of L steps may need of either kind (checked afterwards)
-    const float ex = floorf(fminf(fmaxf(e0 + e1 * (float)L, 0.0f), (float)L));
-    const float nvx = ex + 1.0f, nvz = (float)L - ex + 1.0f;
+    // Iterations left before the next mip switch and before z passes z_far.
+    // z, dz = 2^dzlog and mapswitch are exact integers below 2^31, and
+    // z <= mapswitch here; a negative distance to z_far ends the line either
+    // way, so the shifts decide exactly as the divisions would.
+    const int zi = (int)w.z;
+    const int n_mip = ((w.mapswitch - zi) >> w.dzlog) + 1;
+    const int n_far = (zfar - zi) >> w.dzlog;
+    if (n_far <= 0) return false;
+    const int n = min(n_mip, n_far);
+    // steps ahead that cannot draw (at least; n when none of the level's can)
+    int hidden = 0;
+    if (SKIP) {
+      bool look = w.ofs >= w.end;
+      for (;;) {
+        if (look) dda_look_ahead(w, sc, lc, hidden, n, lane);
+        const int at = max(w.ofs, 0) / kSkipSteps;  // the group of the next step
+        const uint64_t vis = uni64(__ballot(!skip_hidden(w.bound, ymin))) >> at;
+        if (vis) {
+          hidden = max((at + (int)__builtin_ctzll(vis)) * kSkipSteps - w.ofs, 0);
+          break;
+        }
+        hidden = w.end - w.ofs;  // to the window's end: look on from there
+        if (hidden >= n || hidden > kSkipReach) break;
+        look = true;
+      }
+    }
+    // The chunk: L steps from T steps on, which begin one step before the
+    // first that may draw.  emit = false: none of them may.
+    int T = max(hidden - 1, 0), L = min(64, n - T);
+    bool emit = true;
+    if (hidden >= n || hidden > kSkipReach) {
+      T = max(min(hidden, n) - 64, 0);
+      L = min(64, min(hidden, n) - T);
+      emit = false;
+    }
+    // Closed form (dda_terms.h): past a line's first chunk, where every
+    // sequence crosses many binades, nearly every chunk's sequences stay in
+    // one or cross into the next one once.
     const bool xseq = (0x0d >> lane) & 1;  // lanes 0, 2, 3
-    const float nv = xseq ? nvx : nvz;
-    DdaTerms q;
-    bool fit = dda_fit_one(w.s, w.g, nv, q);
-    if ((__ballot(fit) & 0x3f) != 0x3f) {
-      DdaTerms q2;
-      const bool fit2 = dda_fit_two(w.s, w.g, nv, q2, HwRcp());
-      if (!fit) q = q2;
-      fit = fit || fit2;
+    bool ok = false;
+    if (w.dnow > 0.0f) {
+      const float sA = readlane_f(w.q.s, 0), sB = readlane_f(w.q.s, 1);
+      const float gA = readlane_f(w.g, 0), gB = readlane_f(w.g, 1);
+      // x crossings among the first t steps: the merge of sA + i*gA and
+      // sB + j*gB, i + j = t, wants A's term i-1 <= B's term j and B's
+      // term j-1 < A's term i, so i = floor((sB - sA + gA + t*gB) / (gA + gB))
+      const float gr = __builtin_amdgcn_rcpf(gA + gB);
+      const float e0 = (sB - sA + gA) * gr, e1 = gB * gr;
+      if (__ballot(w.q.rem < 0.0f) & 0x3f) w.q = dda_fit(w.q.s, w.g, HwRcp());
+      for (;;) {
+        // terms the chunk may need of either kind (checked afterwards)
+        const float n_steps = (float)(T + L);
+        const float ex = floorf(fminf(fmaxf(e0 + e1 * n_steps, 0.0f), n_steps));
+        const float nv = (xseq ? ex : n_steps - ex) + 1.0f;
+        DdaTerms q{w.q.s, w.q.G, w.q.s, w.q.G, w.q.rem, w.q.rem};
+        if (__ballot(nv > w.q.rem) & 0x3f) q = dda_terms(w.q, w.g, HwRcp());
+        ok = !(__ballot(nv > q.last) & 0x3f) && dda_merge(w, c, q, T, L, e0, e1, xseq, dl, lane);
+        if (!SKIP || ok || T == 0) break;
+        // too many binades on the way: half of it, or one chunk from here
+        if (T >= 128) {
+          T >>= 1;
+          L = 64;
+          emit = false;
+        } else {
+          T = 0;
+          L = min(64, n);
+          emit = hidden < L;
+        }
+      }
+    } else {
+      T = 0;
+      L = min(64, n);
+      emit = hidden < L;
     }
-    ok = (__ballot(fit) & 0x3f) == 0x3f &&
-         dda_merge(w, c, q, L, e0, e1, nvx, nvz, xseq, dl, lane);
+    if (!ok) dda_chain(w, c, L, dl, lane);
+    w.z += (float)(T + L) * w.dz;
+    if (SKIP) w.ofs += T + L;
+    if (emit) {
+      c.L = L;
+      c.mip = w.mip;
+      c.shift = w.shift;
+      c.slab = w.slab;
+      return true;
+    }
   }
-  if (!ok) dda_chain(w, c, L, dl, lane);
-  w.z += (float)L * w.dz;
-  return true;
 }
 
 // Cell of each step of the chunk just walked (Cuda_Render.h:416-442) and the
@@ -505,7 +618,7 @@ __device__ inline void dda_gather(const DdaWalk& w, DdaChunk& c, float vpx, floa
   const int vx = (voxel_x >> w.mip) & (w.gridx - 1);
   const int vz = (voxel_z >> w.mip) & (w.gridz - 1);
   c.ent = make_uint2(0u, 0u);
-  if (lane < c.L) c.ent = w.map[vx + vz * w.gridx];
+  if (lane < c.L && lane >= c.first) c.ent = w.map[vx + vz * w.gridx];
 }
 
 // Chunks handed from the producer wavefront (DDA + pointer gather) to the
@@ -516,7 +629,9 @@ struct ChunkRing {
   uint2 ent[3][64];
   const uint16_t* slab[3];
   int L[3], mip[3], shift[3], have[3];
-  int stop[3];  // written by the consumer in the round that uses the slot
+  // written by the consumer in the round that uses the slot
+  int stop[3], horizon[3];
+  LineConsts lc;  // the producer's
 };
 
 // The fields the consumer reads: distances, level and the gathered entry.
@@ -552,12 +667,12 @@ __device__ inline void ring_get(const ChunkRing& r, int s, DdaChunk& c, int lane
 // steps often show several elements, as in grazing views of caved terrain;
 // the persistent batch kernel leaves it off, where its registers spill).
 // LDS arguments: bits = the line's bitmap, dl = DDA scratch, rc = run cache,
-// sweep_lds = 64 ints for the horizon sweep followed by kWalkEndWords words
-// for the early-end test's constants.
+// sweep_lds = 64 ints for the horizon sweep followed by kLineConstWords words
+// for the line's constants.
 template <bool COUNT, bool TWO = false, bool PAR_ELEMS = true, int RC = kRunCache>
 __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_raymap& rm,
                                         uint32_t* __restrict__ row, int32_t* __restrict__ clip,
-                                        uint32_t* bits, float* dl, uint16_t* rc, int* sweep_lds,
+                                        uint32_t* bits, float* dl, lds_u16* rc, int* sweep_lds,
                                         unsigned long long* counts, ChunkRing* ring = nullptr) {
   static_assert(!(COUNT && TWO), "the counting variant walks with one wavefront");
   const int lane = threadIdx.x & 63;
@@ -678,10 +793,11 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     const float i0x = g0x * frac_x, i0y = g0y * frac_x, i1x = g1x * frac_y, i1y = g1y * frac_y;
     const float gv[6] = {sqrtf(g0x * g0x + g0y * g0y), sqrtf(g1x * g1x + g1y * g1y), g0x, g0y, g1x, g1y};
     const float sv[6] = {sqrtf(i0x * i0x + i0y * i0y), sqrtf(i1x * i1x + i1y * i1y), i0x, i0y, i1x, i1y};
-    wk.s = wk.g = 0;
+    wk.q = DdaSeq{0.0f, 0.0f, -1.0f};
+    wk.g = 0;
 #pragma unroll
     for (int j = 0; j < 6; j++) {
-      wk.s = lane == j ? sv[j] : wk.s;
+      wk.q.s = lane == j ? sv[j] : wk.q.s;
       wk.g = lane == j ? gv[j] : wk.g;
     }
   }
@@ -702,14 +818,19 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
   const float y_add = uni_f((vertical ? cos_x : 0.0f) * hmul);
   const int zfar = uni(rm.far_distance);
   const float mountain = vpy;
-  // the early-end test's constants, in LDS behind the sweep marks
-  WalkEnd* wend = reinterpret_cast<WalkEnd*>(sweep_lds + 64);
-  float wfloor = 0.0f;  // held in a scalar register across the walk
-  if (!producer) {
-    if (lane == 0) wend->init(cos_x, sin_x, hmul, ray_x, ray_z, vertical, mountain, half);
-    wave_sync();
-    wfloor = uni_f(wend->floor_());
+  wk.bound = 0;
+  wk.ofs = wk.end = 0;
+  // the line's constants, in LDS behind the sweep marks (the producer of a
+  // two-wavefront line has its own)
+  LineConsts* lc = reinterpret_cast<LineConsts*>(sweep_lds + 64);
+  if (producer) lc = &ring->lc;
+  const WalkEnd* wend = &lc->end;
+  if (lane == 0) {
+    lc->end.init(cos_x, sin_x, hmul, ray_x, ray_z, vertical, mountain, half);
+    lc->line.init(ddx, ddy, vpx, vpz);
   }
+  wave_sync();
+  const float wfloor = uni_f(wend->floor_());  // held in a scalar register across the walk
 
   // Software pipeline: while chunk c's run-cache loads are in flight the DDA
   // of chunk c+1 runs, and while chunk c is replayed the pointer-map gather
@@ -793,35 +914,29 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     const bool cand = valid && F > ymin && !culled0;
     const uint64_t rc_base = wofs & ~(uint64_t)7;  // 16-byte aligned start
     const int rc_delta = (int)(wofs - rc_base);
-    const uint16_t* cached = rc + lane * RC + rc_delta;
+    const RcColumn cached{rc, lane, rc_delta};
     const int ccap = cand ? RC - rc_delta : 0;
     static_assert(RC % 8 == 0 && RC >= 24, "the run cache is fetched in 16-byte words");
     constexpr int kWords = RC / 8;
-    typedef unsigned int rc_word __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(1))) const rc_word g_rc_word;
-    rc_word rcw[kWords];  // loaded and stored only for candidates
+    // A wait for this wavefront's LDS reads (the last chunk's, of the cache)
+    // before the loads may write it, and for the loads before it is read.
+    constexpr int kWaitLds = 0xc07f, kWaitLoads = 0x0f70;  // lgkmcnt(0), vmcnt(0)
     if (cand) {
-      // Global loads: in the drawing wavefront of a two-wavefront line the
-      // slab pointer comes through LDS, and flat loads would make each LDS
-      // wait until they return wait for them too.
-      const g_rc_word* src = (const g_rc_word*)(slab + rc_base);
+      typedef __attribute__((address_space(1))) const void g_void;
+      typedef __attribute__((address_space(3))) void l_void;
+      __builtin_amdgcn_s_waitcnt(kWaitLds);
+      const uint16_t* src = slab + rc_base;
 #pragma unroll
-      for (int i = 0; i < kWords; i++) rcw[i] = src[i];
+      for (int i = 0; i < kWords; i++)
+        __builtin_amdgcn_global_load_lds((g_void*)(src + 8 * i), (l_void*)(rc + 512 * i), 16, 0, 0);
     }
 
     // ---- next chunk's DDA (the run cache loads are in flight meanwhile)
-    if constexpr (decltype(produce)::value) have_next = dda_next_chunk(wk, nxt, sc, zfar, dl, lane);
+    if constexpr (decltype(produce)::value) have_next = dda_next_chunk<!COUNT>(wk, nxt, sc, *lc, zfar, ymin, dl, lane);
 
-    // The stores wait for the loads: a walking wavefront stores after the DDA
-    // above, a drawing-only one after the span parameters below.
-    auto store_rc = [&]() {
-      if (cand) {
-        rc_word* dst = reinterpret_cast<rc_word*>(rc + lane * RC);
-#pragma unroll
-        for (int i = 0; i < kWords; i++) dst[i] = rcw[i];
-      }
-    };
-    if constexpr (decltype(produce)::value) store_rc();
+    // A walking wavefront waits for the cache before the gather below goes
+    // out, a drawing-only one after the span parameters.
+    if constexpr (decltype(produce)::value) __builtin_amdgcn_s_waitcnt(kWaitLoads);
     // ---- next chunk's pointer gather: in flight during this chunk's replay
     if constexpr (decltype(produce)::value) {
       if (have_next) dda_gather(wk, nxt, vpx, vpz, fix_xf, fix_yf, lane);
@@ -856,7 +971,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
         onedz2F /= s2r - s1rF;
       }
     }
-    if constexpr (!decltype(produce)::value) store_rc();
+    if constexpr (!decltype(produce)::value) __builtin_amdgcn_s_waitcnt(kWaitLoads);
     wave_sync();  // run cache filled
     if (cand) {  // F2: projected top of the next element the loop tests
       int yg = ygF;
@@ -956,7 +1071,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
               const uint64_t wofs = (uint64_t)aofs << shift;
               const int tdelta = (int)(wofs & 7u);
               const int cw = 2 + (int)alen + tdelta + (int)u;
-              const uint32_t col = cw < RC ? rc[a * RC + cw]
+              const uint32_t col = cw < RC ? rc[rc_index(a, cw)]
                                                   : slab[2 + wofs + alen + u];
               row[ymin + lane] = col + (depth << 16);
             }
@@ -995,7 +1110,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
       const uint16_t* tcol = truns + tslen;
       const bool tcached = readlane_i((int)cand, t) != 0;
       const int tdelta = (int)(tofs & 7u);
-      const uint16_t* tcache = rc + t * RC + tdelta;
+      const RcColumn tcache{rc, t, tdelta};
       const int tcap = tcached ? RC - tdelta : 0;
       const float tpz = readlane_f(pz, t), tpy = readlane_f(py3, t);
       const float tczz = readlane_f(czz, t), tcyy = readlane_f(cyy, t);
@@ -1225,7 +1340,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     }
     // ---- early end of the walk (WalkEnd): later steps lie beyond this
     // chunk's last crossing distance
-    if (!done && !cnt.ended && wfloor < (float)ymin + (1.0f - WalkEnd::kAbs) &&
+    if (!done && L > 0 && !cnt.ended && wfloor < (float)ymin + (1.0f - WalkEnd::kAbs) &&
         wend->done(readlane_f(cur.dn, L - 1), ymin, sc.mip[mip].top, sc.sy)) {
       if (COUNT) cnt.end_walk();  // the counting variant walks on to count the reference's work
       else done = true;
@@ -1233,9 +1348,15 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     return !done;
   };
   if constexpr (!TWO) {
+    // the first step has no chunk of its own (L = 0) and only walks ahead
     DdaChunk cur, nxt;
-    bool have = dda_next_chunk(wk, cur, sc, zfar, dl, lane);
-    if (have) dda_gather(wk, cur, vpx, vpz, fix_xf, fix_yf, lane);
+    cur.L = 0;
+    cur.mip = 0;
+    cur.shift = 0;
+    cur.slab = wk.slab;
+    cur.db = cur.dn = 0.0f;
+    cur.ent = make_uint2(0u, 0u);
+    bool have = true;
     const std::true_type yes;
     while (have && chunk_step(yes, cur, nxt, have)) {
       // the copy waits for the gather, whose entries the next step starts with
@@ -1264,7 +1385,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
       int s = 0, s1 = 2, s2 = 1;  // slots of chunks n, n-1, n-2
       for (int n = 0;; n++) {
         if (n >= 2 && !uni(r.have[s2])) break;
-        more = more && dda_next_chunk(wk, p, sc, zfar, dl, lane);
+        more = more && dda_next_chunk<true>(wk, p, sc, *lc, zfar, ymin, dl, lane);
         ring_put_dda(r, s, p, more, lane);
         if (pend) r.ent[s1][lane] = ent;  // waits for the gather
         if (more) {
@@ -1273,7 +1394,10 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
         }
         pend = more;
         if (n >= 1) __syncthreads();
-        if (n >= 2 && uni(r.stop[s2])) break;
+        if (n >= 2) {
+          if (uni(r.stop[s2])) break;
+          ymin = uni(r.horizon[s2]);
+        }
         s2 = s1;
         s1 = s;
         s = s == 2 ? 0 : s + 1;
@@ -1290,7 +1414,10 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
         const bool more = chunk_step(no, cur, unused, hu);
         // A slot's flag is read after this round's barrier and rewritten
         // three rounds later, so no wavefront can see a later round's value.
-        if (lane == 0) r.stop[s] = more ? 0 : 1;
+        if (lane == 0) {
+          r.stop[s] = more ? 0 : 1;
+          r.horizon[s] = ymin;
+        }
         __syncthreads();
         if (uni(r.stop[s])) break;
         s = s == 2 ? 0 : s + 1;

@@ -14,8 +14,8 @@
 
 using namespace rlevox;
 
-// Nonzero only in the planted build: accepts a first step that differs from
-// the later ones, as a tie leaves it.
+// Nonzero only in the planted build: takes the first step for all of the
+// binade, though a tie may have rounded it the other way.
 #ifndef DDA_TERMS_PLANT
 #define DDA_TERMS_PLANT 0
 #endif
@@ -28,21 +28,29 @@ struct Rcp {
 static long tried = 0, one = 0, two = 0, bad = 0;
 
 static void check(float s, float g, int n, float ulps) {
-  DdaTerms q;
   tried++;
-  bool ok = dda_fit_one(s, g, (float)n, q);
-  if (DDA_TERMS_PLANT && !ok)
-    ok = dda_same_binade(s, fmaf((float)n, q.G, s));
-  if (ok) one++;
-  else if (dda_fit_two(s, g, (float)n, q, Rcp{ulps})) {
-    ok = true;
+  const Rcp rcp{ulps};
+  DdaSeq q = dda_fit(s, g, rcp);
+  if (DDA_TERMS_PLANT == 1 && q.rem >= 0.0f && dda_same_binade(s, fmaf((float)n, q.G, s)))
+    q.rem = (float)n;  // as if no tie could be
+  DdaTerms w = dda_terms(q, g, rcp);
+  if (q.rem >= (float)n) {
+    one++;
+    w.K = w.last = q.rem;
+  } else if (w.last >= (float)n) {
     two++;
+  } else {
+    return;
   }
-  if (!ok) return;
   float t = s;
   for (int k = 0; k <= n; k++) {
-    const float v = dda_term(q, (float)k);
-    if (dda_bits(v) != dda_bits(t)) {
+    const float v = dda_term(w, (float)k);
+    const DdaSeq a = dda_advance(w, (float)k);  // and the walk that goes on from there
+    float u = t;
+    bool same = dda_bits(v) == dda_bits(t) && dda_bits(a.s) == dda_bits(t);
+    for (int j = 0; same && j <= 3 && (float)j <= a.rem; j++, u = u + g)
+      same = dda_bits(fmaf((float)j, a.G, a.s)) == dda_bits(u);
+    if (!same) {
       if (bad++ < 5) std::printf("s %a g %a n %d term %d: %a, sum %a\n", s, g, n, k, v, t);
       return;
     }
@@ -53,7 +61,7 @@ static void check(float s, float g, int n, float ulps) {
 int main() {
   std::mt19937_64 rng(11);
   std::uniform_real_distribution<double> U(0.0, 1.0);
-  auto len = [&] { return 1 + (int)(U(rng) * 64); };
+  auto len = [&] { return 1 + (int)(U(rng) * (U(rng) < 0.2 ? 1024 : 64)); };
   auto ulps = [&] { return (float)((int)(U(rng) * 5) - 2); };
   for (int ln = 0; ln < 20000; ln++) {  // the six sequences of a line, chunk by chunk
     const double ang = U(rng) * 6.283185307179586;
