@@ -615,14 +615,63 @@ struct GapTile {
   uint2 p[kGapTH][kGapTW];
 };
 
+// The tap word of colour16 in bits 0-15 of c, or (HIGH) in bits 16-31: one
+// byte permute.
+template <bool HIGH>
 __device__ inline uint32_t gap_word(uint32_t c) {
-  return (c & 0xffu) | (1u << 16) | ((c >> 8) << 24);
+  return __builtin_amdgcn_perm(c, 1u, HIGH ? 0x07000c06u : 0x05000c04u);
 }
 
 // The hardware reciprocal (v_rcp_f32, at most 1 ulp off) for recip_div.h.
 struct HwRcp {
   __device__ float operator()(float x) const { return __builtin_amdgcn_rcpf(x); }
 };
+
+// The tap offsets of one axis, floor(((2a-5) r + 640) / 1280) for a = 0..4,
+// by the radius r = floor(78720 / dmin):
+//   r <= 128  {0, 0, 0, 0, 0}: every tap is the pixel itself, so its shade
+//             stays (26 s + 13) / 26 = s, or too few taps qualify
+//   r <= 213  {-1, 0, 0, 0, 0}
+//   r <= 384  {-1, -1, 0, 0, 1}
+//   r <= 639  {-2, -1, 0, 0, 1}
+// and spread over five columns above.  r <= R is dmin > floor(78720 / (R+1)).
+// So pixels beyond kGapFar keep their colour, and nearer ones up to kGap4
+// need 2x2, 3x3 or 4x4 taps with small weights in place of 5x5 (a wavefront
+// takes the number its nearest pixel needs).  The pass issues instructions
+// for most of its time (14 of 20.5 us at 1080p, 60 of 72 us at 4K were
+// VALU issue): 25 taps took three instructions and an LDS read each.
+constexpr int kGapFar = 610, kGap2 = 367, kGap3 = 204, kGap4 = 123;
+
+// Taps at offsets 2-N..1 (N = 2: -1 and 0) of both axes, weighted per lane by
+// the lane's own class; returns the weighted sum of the qualifying tap words.
+template <int N>
+__device__ inline uint32_t gap_taps(const uint2* tp, int centre, int dmin, int dlim) {
+  constexpr int kLo = N == 2 ? -1 : 2 - N;
+  uint32_t w[N];  // of offset kLo + i
+  if (N == 2) {
+    w[0] = 1;
+    w[1] = 4;
+  } else {
+    const bool c2 = dmin > kGap2, c4 = dmin <= kGap3;  // 2x2, 4x4 lanes
+    w[N - 3] = c2 | c4 ? 1 : 2;  // -1
+    w[N - 2] = c2 ? 4 : 2;       // 0
+    w[N - 1] = c2 ? 0 : 1;       // 1
+    if (N == 4) w[0] = c4 ? 1 : 0;
+  }
+  uint32_t acc = 0;
+#pragma unroll
+  for (int b = 0; b < N; b++) {  // rows: an offset points up the image
+    uint32_t r = 0;
+#pragma unroll
+    for (int a = 0; a < N; a++) {
+      const uint2 q = tp[centre - (kLo + b) * kGapTW + kLo + a];
+      // 24-bit products: the count and the shade; the high byte is not needed
+      r += __umul24((int)q.x <= dlim ? q.y : 0u, w[a]);
+    }
+    acc += __umul24(r, w[b]);
+  }
+  return acc;
+}
 
 __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ cin_,
                                     const int32_t* __restrict__ dep_, uint16_t* __restrict__ cout_,
@@ -657,10 +706,10 @@ __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ c
       if (i < kQuads) {
         const int ty = i / kQ, tq = i - ty * kQ;
         uint4* dst = reinterpret_cast<uint4*>(&t.p[ty][4 * tq]);
-        dst[0] = make_uint4((uint32_t)dv[k].x, gap_word(cv[k].x & 0xffffu), (uint32_t)dv[k].y,
-                            gap_word(cv[k].x >> 16));
-        dst[1] = make_uint4((uint32_t)dv[k].z, gap_word(cv[k].y & 0xffffu), (uint32_t)dv[k].w,
-                            gap_word(cv[k].y >> 16));
+        dst[0] = make_uint4((uint32_t)dv[k].x, gap_word<false>(cv[k].x), (uint32_t)dv[k].y,
+                            gap_word<true>(cv[k].x));
+        dst[1] = make_uint4((uint32_t)dv[k].z, gap_word<false>(cv[k].y), (uint32_t)dv[k].w,
+                            gap_word<true>(cv[k].y));
       }
     }
   } else {
@@ -684,7 +733,7 @@ __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ c
       const int i = threadIdx.x + k * 256;
       if (i < kGapTW * kGapTH) {
         const int ty = i / kGapTW, tx = i - ty * kGapTW;
-        t.p[ty][tx] = make_uint2((uint32_t)dv[k], gap_word(cv[k]));
+        t.p[ty][tx] = make_uint2((uint32_t)dv[k], gap_word<false>(cv[k]));
       }
     }
   }
@@ -696,28 +745,36 @@ __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ c
     int dmin = (int)ctr.x;
     for (int k = 0; k < 7; k++) dmin = min(dmin, (int)t.p[ly - kRingDy[k]][lx + kRingDx[k]].x);
     uint16_t out = (uint16_t)((ctr.y & 0xffu) | ((ctr.y >> 24) << 8));  // the pixel's colour
-    if (dmin < RLEVOX_SKY_DEPTH) {
-      const int dm = max(dmin, 1);
-      const int r_q8 = div_78720(dm, HwRcp());  // floor(78720 / dm)
-      if (r_q8 >= 42) {
+    if (dmin <= kGapFar) {
+      // A tap qualifies when 10*dmin >= 7*d, i.e. d <= floor(10*dmin/7)
+      // (below the sky depth).  The centre pixel counts once with its own
+      // shade.
+      const int dlim = (10 * dmin) / 7;
+      const uint2* tp = &t.p[0][0];
+      const int centre = ly * kGapTW + lx;
+      uint32_t acc = ctr.y;
+      bool taps = true;
+      if (!__any(dmin <= kGap2)) {
+        acc += gap_taps<2>(tp, centre, dmin, dlim);
+      } else if (!__any(dmin <= kGap3)) {
+        acc += gap_taps<3>(tp, centre, dmin, dlim);
+      } else if (!__any(dmin <= kGap4)) {
+        acc += gap_taps<4>(tp, centre, dmin, dlim);
+      } else {
+        const int r_q8 = div_78720(max(dmin, 1), HwRcp());  // floor(78720 / dmin)
         // tap offsets floor(((2a-5) r + 640) / 1280); the numerators stay
         // above -655360, so a bias of 512*1280 keeps the division unsigned
         int o[5];
 #pragma unroll
         for (int a = 0; a < 5; a++)
           o[a] = (int)((uint32_t)((2 * a - 5) * r_q8 + 640 + 655360) / 1280u) - 512;
-        if (o[0] >= -kGapHalo) {
-          // r_q8 >= 42 means dmin <= 1874: a tap qualifies when
-          // 10*dmin >= 7*d, i.e. d <= floor(10*dmin/7) (below the sky depth).
+        taps = o[0] >= -kGapHalo;
+        if (taps) {
           // Branch-free: every tap is read (so the 25 LDS reads can be in
-          // flight together) and a failing tap adds 0.  The centre pixel
-          // counts once with its own shade.
-          const int dlim = (10 * dmin) / 7;
-          uint32_t acc = ctr.y;
+          // flight together) and a failing tap adds 0.
           int rowo[5];
 #pragma unroll
           for (int b = 0; b < 5; b++) rowo[b] = (ly - o[b]) * kGapTW + lx;
-          const uint2* tp = &t.p[0][0];
 #pragma unroll
           for (int a = 0; a < 5; a++) {
 #pragma unroll
@@ -726,13 +783,13 @@ __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ c
               acc += (int)q.x <= dlim ? q.y : 0u;
             }
           }
-          const int n = (int)((acc >> 16) & 0xffu), sum = (int)(acc & 0xffffu);
-          // n <= 26, sum + n/2 <= 26 * 255 + 13
-          if (n > 6) out = (uint16_t)((out & 0xff00) | div_small(sum + n / 2, n, HwRcp()));
         } else {
           out = gapfill_pixel(W, H, cin, dep, x, prow);
         }
       }
+      const int n = (int)((acc >> 16) & 0xffu), sum = (int)(acc & 0xffffu);
+      // n <= 26, sum + n/2 <= 26 * 255 + 13
+      if (taps && n > 6) out = (uint16_t)((out & 0xff00) | div_small(sum + n / 2, n, HwRcp()));
     }
     *((g_u16_out*)cout_ + ((uint32_t)prow * (uint32_t)W + (uint32_t)x)) = out;
   }
