@@ -49,11 +49,17 @@ __device__ inline int find_view(const ViewDesc* __restrict__ v, int n, int64_t g
 // unless the tuning says otherwise.  RC: LDS run-cache words per column.
 template <bool PAR, int RC>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_raycast_batch(BatchHeader* __restrict__ h,
-                                                      const ViewDesc* __restrict__ views) {
+                                                      const ViewDesc* __restrict__ views_) {
   __shared__ uint32_t bits[(RLEVOX_MAX_RS + 31) / 32];
   __shared__ uint4 rcache[64 * RC / 8];
   __shared__ int sweep[64 + kLineConstWords];
   __shared__ __align__(16) float dda[kDdaLds];
+  // The descriptors as constant memory: the line's fields come by scalar
+  // loads.  As vector loads they held registers across the walk and the
+  // level table was read with flat loads.
+  typedef const RLEVOX_CONST_AS ViewDesc c_view;
+  typedef const RLEVOX_CONST_AS SceneDev c_scene;
+  c_view* views = (c_view*)views_;
   const int lane = threadIdx.x;
   const int64_t total = h->total_lines;
   const int nv = h->nviews;
@@ -64,10 +70,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     g = (uint32_t)__builtin_amdgcn_readlane((int)g, 0);
     if ((int64_t)g >= total) break;
     while (v + 1 < nv && views[v + 1].line_begin <= (int64_t)g) v++;
-    const ViewDesc& vd = views[v];
+    const c_view& vd = views[v];
     // lines of a view from the last to the first, as the single-view kernels
     const int x = vd.rm.map_line_count - 1 - (int)((int64_t)g - vd.line_begin);
-    render_line_wave<false, false, PAR, RC>(x, *vd.scene, vd.rm,
+    render_line_wave<false, false, PAR, RC>(x, *(c_scene*)vd.scene, vd.rm,
                                           vd.raybuf + (size_t)x * (size_t)vd.rm.rs,
                             vd.clip + 2 * x, bits, dda, (lds_u16*)rcache,
                             sweep, nullptr);
@@ -143,14 +149,16 @@ __global__ __launch_bounds__(256) void k_compose_batch(BatchHeader* __restrict__
       int32_t d;
       compose_pixel(vd.rm, vd.raybuf, vd.clip, px, row, ct.col[threadIdx.x & 63],
                     ct.row[threadIdx.x >> 6], ct.border, c, d);
-      uint16_t* out = (vd.post & RLEVOX_POST_GAPFILL) ? vd.ctmp : vd.colour;
-      out[(size_t)row * W + px] = c;
-      vd.depth[(size_t)row * W + px] = d;
+      typedef __attribute__((address_space(1))) int32_t g_i32_out;
+      g_u16_out* out = (g_u16_out*)((vd.post & RLEVOX_POST_GAPFILL) ? vd.ctmp : vd.colour);
+      const uint32_t i = (uint32_t)row * (uint32_t)W + (uint32_t)px;  // W, H <= 8192
+      out[i] = c;
+      ((g_i32_out*)vd.depth)[i] = d;
     }
   }
 }
 
-__global__ __launch_bounds__(256) void k_gapfill_batch(BatchHeader* __restrict__ h,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_gapfill_batch(BatchHeader* __restrict__ h,
                                                        const ViewDesc* __restrict__ views) {
   __shared__ GapTile gt;
   __shared__ int64_t next[2];

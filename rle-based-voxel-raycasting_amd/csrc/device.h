@@ -39,15 +39,20 @@ struct SceneDev {
 // Ray-buffer line bitmap words for render size rs.
 __host__ __device__ inline int bitmap_words(int rs) { return (rs + 31) >> 5; }
 
-// Saturating float -> int32 with NaN -> 0, branch-free: NaN is replaced
-// first, the median-of-three clamps to [-2^31, 2^31 - 128] (the largest float
-// below 2^31), where the conversion is exact truncation, and values from 2^31
-// up select INT32_MAX.
+// Saturating float -> int32 with NaN -> 0: what v_cvt_i32_f32 does by itself
+// (a C++ conversion is undefined out of range, so the compiler may not be
+// asked for it; clamped by hand it took six instructions).  The result
+// counts as different from lane to lane: callers with uniform values say so.
 __device__ inline int d_f2i(float f) {
-  const float g = f != f ? 0.0f : f;
-  const int r = (int)__builtin_amdgcn_fmed3f(g, -2147483648.0f, 2147483520.0f);
-  return g >= 2147483648.0f ? INT32_MAX : r;
+  int r;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(f));
+  return r;
 }
+
+// The lanes (of those active) for which p holds.  The builtin takes a
+// compare's mask as it is; __ballot's int argument made every mask go
+// through a register and a second compare.
+__device__ inline uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
 // LDS bitmap of one line, word w of this lane at base[w * stride].
 struct LineBits {
@@ -60,11 +65,31 @@ struct LineBits {
   }
 };
 
+// Global-memory views: the kernels read these pointers from descriptors,
+// from structures and through LDS, where the compiler would emit flat
+// accesses, which wait on both counters and for each other.
+typedef __attribute__((address_space(1))) const int32_t g_i32;
+typedef __attribute__((address_space(1))) const uint16_t g_u16;
+typedef int v4i32 __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u32 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(1))) const v4i32 g_v4i32;
+typedef __attribute__((address_space(1))) const v2u32 g_v2u32;
+typedef __attribute__((address_space(1))) uint16_t g_u16_out;
+typedef __attribute__((address_space(1))) uint32_t g_u32_out;
+typedef __attribute__((address_space(1))) const v2u32 g_entry;  // a pointer-map entry
+
+// Descriptors that no kernel writes, read as constant memory: uniform fields
+// come by scalar loads into scalar registers.
+#define RLEVOX_CONST_AS __attribute__((address_space(4)))
+
 struct F3 {
   float x, y, z;
 };
 __device__ inline F3 f3(float x, float y, float z) { return F3{x, y, z}; }
-__device__ inline F3 f3ld(const float* p) { return F3{p[0], p[1], p[2]}; }
+template <class P>
+__device__ inline F3 f3ld(const P& p) {
+  return F3{p[0], p[1], p[2]};
+}
 __device__ inline F3 operator+(F3 a, F3 b) { return f3(a.x + b.x, a.y + b.y, a.z + b.z); }
 __device__ inline F3 operator-(F3 a, F3 b) { return f3(a.x - b.x, a.y - b.y, a.z - b.z); }
 __device__ inline F3 operator*(F3 a, float s) { return f3(a.x * s, a.y * s, a.z * s); }
@@ -80,7 +105,8 @@ __device__ inline float line_scale(F3 in, F3 ctr, float cmax, float cmin) {
 }
 
 // MatMul (Cuda_Render.h:67-73), row-vector convention.
-__device__ inline F3 mat_apply(const float (*m)[4], F3 v) {
+template <class M>
+__device__ inline F3 mat_apply(const M& m, F3 v) {
   return f3(m[0][0] * v.x + m[1][0] * v.y + m[2][0] * v.z + m[3][0],
             m[0][1] * v.x + m[1][1] * v.y + m[2][1] * v.z + m[3][1],
             m[0][2] * v.x + m[1][2] * v.y + m[2][2] * v.z + m[3][2]);
@@ -553,16 +579,6 @@ __device__ inline void compose_pixel(const rlevox_raymap& rm, const uint32_t* __
 __constant__ const int kRingDx[7] = {0, 9, 9, 2, -8, -10, -3};
 __constant__ const int kRingDy[7] = {10, 6, -4, -10, -7, 3, 10};
 
-// Global-memory views of the gap-fill's buffers: the batch kernels read the
-// pointers from a view descriptor, where the compiler would emit flat loads.
-typedef __attribute__((address_space(1))) const int32_t g_i32;
-typedef __attribute__((address_space(1))) const uint16_t g_u16;
-typedef int v4i32 __attribute__((ext_vector_type(4)));
-typedef uint32_t v2u32 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(1))) const v4i32 g_v4i32;
-typedef __attribute__((address_space(1))) const v2u32 g_v2u32;
-typedef __attribute__((address_space(1))) uint16_t g_u16_out;
-
 __device__ inline int floor_div_pos(int a, int b) {  // b > 0
   const int q = a / b, r = a % b;
   return (r != 0 && r < 0) ? q - 1 : q;
@@ -754,11 +770,11 @@ __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ c
       const int centre = ly * kGapTW + lx;
       uint32_t acc = ctr.y;
       bool taps = true;
-      if (!__any(dmin <= kGap2)) {
+      if (ballot(dmin <= kGap2) == 0) {
         acc += gap_taps<2>(tp, centre, dmin, dlim);
-      } else if (!__any(dmin <= kGap3)) {
+      } else if (ballot(dmin <= kGap3) == 0) {
         acc += gap_taps<3>(tp, centre, dmin, dlim);
-      } else if (!__any(dmin <= kGap4)) {
+      } else if (ballot(dmin <= kGap4) == 0) {
         acc += gap_taps<4>(tp, centre, dmin, dlim);
       } else {
         const int r_q8 = div_78720(max(dmin, 1), HwRcp());  // floor(78720 / dmin)

@@ -60,9 +60,14 @@ struct SkipBase {  // the last step taken, and what follows it
     return fmaxf(fmaxf(a, b), dnow);
   }
 };
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(1))) const int32_t skip_tops;  // read as global memory
+#else
+typedef const int32_t skip_tops;
+#endif
 struct SkipLevel {
   int mip, gridx, gridz;
-  const int32_t* tops;  // per block: highest run top (world row), x fastest
+  skip_tops* tops;  // per block: highest run top (world row), x fastest
   int top;              // highest run top of the level and all coarser ones
 };
 

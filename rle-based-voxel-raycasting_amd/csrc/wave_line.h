@@ -98,7 +98,8 @@ typedef __attribute__((address_space(3))) uint16_t lds_u16;
 struct RcColumn {
   const lds_u16* rc;
   int lane, delta;
-  __device__ uint16_t operator[](int i) const { return rc[rc_index(lane, delta + i)]; }
+  __device__ int index(int i) const { return rc_index(lane, delta + i); }
+  __device__ uint16_t operator[](int i) const { return rc[index(i)]; }
 };
 
 // LDS floats per wavefront used by the DDA chunk.
@@ -108,7 +109,7 @@ constexpr int kDdaLds = 6 * 68 + 64;
 __device__ inline int first_clear(const uint32_t* bits, int from, int to, int lane) {
   for (int base = from; base < to; base += 64) {
     const int y = base + lane;
-    const uint64_t m = uni64(__ballot(y < to && !lds_bit(bits, y)));
+    const uint64_t m = uni64(ballot(y < to && !lds_bit(bits, y)));
     if (m) return uni(base + __builtin_ctzll(m));
   }
   return to;
@@ -178,11 +179,29 @@ __device__ inline void bits_or(uint32_t* bits, int base, uint64_t m, int lane) {
   }
 }
 
+// Slab word of a column: from the run cache (at rc[index]) where it holds the
+// word, else from memory.  Nearly always it holds every lane's, and that way
+// is kept apart, uniformly, until the word has arrived (the empty asm reads
+// it): joined earlier, it would wait for the memory load's counter, and with
+// it for every store the wavefront has in flight (one counter for both).
+__device__ inline uint32_t column_word(bool cached, const lds_u16* rc, int index, g_u16* mem) {
+  uint32_t w;
+  if (ballot(!cached) == 0) {
+    w = rc[index];
+    asm volatile("" : "+v"(w));
+  } else {
+    if (cached) w = rc[index];
+    else w = *mem;
+    asm volatile("" : "+v"(w));
+  }
+  return w;
+}
+
 // Draws pixels [y0, s2) of one span (uniform arguments; Cuda_Render.h:
 // 678-733).  Pixel y0+k has had k per-pixel increments.
 __device__ inline int draw_span(int y0, int s2, float uzb, float ozb, float u2dz, float onedz2,
                                 float tlo, float thi, RcColumn cached, int ccap,
-                                const uint16_t* colours, int cofs, uint32_t* __restrict__ row,
+                                g_u16* colours, int cofs, g_u32_out* row,
                                 uint32_t* bits, int lane) {
   int drawn = 0;
   for (int base = y0; base < s2; base += 64) {
@@ -199,10 +218,9 @@ __device__ inline int draw_span(int y0, int s2, float uzb, float ozb, float u2dz
       const uint32_t u = (uint32_t)d_f2i(fu);
       const uint32_t depth = (uint32_t)d_f2i(1.0f / oz) & 0xfffeu;
       const int cw = cofs + (int)u;
-      const uint32_t col = cw < ccap ? cached[cw] : colours[u];
-      row[y] = col + (depth << 16);
+      row[y] = column_word(cw < ccap, cached.rc, cached.index(cw), colours + u) + (depth << 16);
     }
-    const uint64_t dm = __ballot(draw);
+    const uint64_t dm = ballot(draw);
     drawn += (int)__popcll(dm);
     bits_or(bits, base, dm, lane);  // pixel base+i is bit i of dm
     wave_sync();
@@ -227,7 +245,7 @@ __device__ inline SpanWindow span_window(const uint32_t* bits, int s1, int e2, i
   SpanWindow w;
   if (e2 - s1 <= 64) {
     const bool clear = lane < e2 - s1 && !lds_bit(bits, s1 + lane);
-    w.m = uni64(__ballot(clear));
+    w.m = uni64(ballot(clear));
     w.y0 = uni(w.m ? s1 + (int)__builtin_ctzll(w.m) : e2);
     w.fused = true;
   } else {
@@ -242,8 +260,8 @@ __device__ inline SpanWindow span_window(const uint32_t* bits, int s1, int e2, i
 // had k per-pixel increments.
 __device__ inline int span_draw(const SpanWindow& w, int s1, int e2, float uzb, float ozb,
                                 float u2dz, float onedz2, float tlo, float thi,
-                                RcColumn cached, int ccap, const uint16_t* colours,
-                                int cofs, uint32_t* __restrict__ row, uint32_t* bits, int lane) {
+                                RcColumn cached, int ccap, g_u16* colours,
+                                int cofs, g_u32_out* row, uint32_t* bits, int lane) {
   if (!w.fused)
     return draw_span(w.y0, e2, uzb, ozb, u2dz, onedz2, tlo, thi, cached, ccap, colours, cofs, row,
                      bits, lane);
@@ -257,8 +275,8 @@ __device__ inline int span_draw(const SpanWindow& w, int s1, int e2, float uzb, 
     const uint32_t u = (uint32_t)d_f2i(fu);
     const uint32_t depth = (uint32_t)d_f2i(1.0f / oz) & 0xfffeu;
     const int cw = cofs + (int)u;
-    const uint32_t col = cw < ccap ? cached[cw] : colours[u];
-    row[s1 + lane] = col + (depth << 16);
+    row[s1 + lane] =
+        column_word(cw < ccap, cached.rc, cached.index(cw), colours + u) + (depth << 16);
   }
   bits_or(bits, s1, w.m, lane);
   wave_sync();
@@ -283,8 +301,8 @@ struct DdaWalk {
   float bound;
   int ofs, end;
   float dz, z, yswitch;
-  const uint2* map;
-  const uint16_t* slab;
+  g_entry* map;
+  g_u16* slab;
 };
 
 // One chunk of up to 64 DDA steps: lane k holds step k and its gathered
@@ -292,7 +310,7 @@ struct DdaWalk {
 struct DdaChunk {
   int L, mip, shift;
   int first;  // lanes below hold no step of the line's own
-  const uint16_t* slab;
+  g_u16* slab;
   float db, dn, pbx, pby;  // per lane: distances and position before the step
   int ib;
   uint2 ent;
@@ -347,14 +365,14 @@ __device__ inline bool dda_merge(DdaWalk& w, DdaChunk& c, const DdaTerms& q, int
         own += few ? 1.0f : (many ? -1.0f : 0.0f);
       }
       const float told = __int_as_float(dpp_move<0x138>(__float_as_int(own), __float_as_int(next)));
-      if (!(__ballot(told != fi) & (~0ull >> (64 - L)))) break;
+      if (!(ballot(told != fi) & (~0ull >> (64 - L)))) break;
       fi = told;
     }
   }
   // the terms after the chunk's last step must still be within the fits
   const float nx = readlane_f(next, L - 1);
   const float n = xseq ? nx : (float)(T + L) - nx;
-  if (__ballot(n > q.last) & 0x3f) return false;
+  if (ballot(n > q.last) & 0x3f) return false;
   const float k = z ? tf - fi : fi;
   const int sx = z ? 4 : 2;
   const float x = term(row[sx], rowK[sx], k);
@@ -430,7 +448,7 @@ __device__ inline void dda_chain(DdaWalk& w, DdaChunk& c, int L, float* dl, int 
   const int rz = lane + cz;
   if (rx < L) slot[rx] = lane;
   if (rz < L) slot[rz] = 64 + lane;
-  const int nx = uni((int)__popcll(__ballot(rx < L)));
+  const int nx = uni((int)__popcll(ballot(rx < L)));
   const int nz = L - nx;
   // The walk's state after the chunk, read in one round trip: the next
   // terms (index nx of the x sequences, nz of the z sequences) and the last
@@ -475,13 +493,14 @@ constexpr int kLineConstWords = (int)(sizeof(LineConsts) / 4);
 
 // The bounds of the window that begins `ahead` steps on, n steps before the
 // next mip switch or the far distance.
-__device__ inline void dda_look_ahead(DdaWalk& w, const SceneDev& sc, const LineConsts& lc,
+template <class Scene>
+__device__ inline void dda_look_ahead(DdaWalk& w, const Scene& sc, const LineConsts& lc,
                                       int ahead, int n, int lane) {
   const float sA = readlane_f(w.q.s, 0), sB = readlane_f(w.q.s, 1);
   const float gA = readlane_f(w.g, 0), gB = readlane_f(w.g, 1);
   const float r = __builtin_amdgcn_rcpf(gA + gB);
   const SkipBase b{w.px, w.py, w.dnow, sA, sB, gA, gB, (sB - sA + gA) * r, gB * r};
-  const SkipLevel v{w.mip, w.gridx, w.gridz, sc.mip[w.mip].tops, sc.mip[w.mip].top};
+  const SkipLevel v{w.mip, w.gridx, w.gridz, (skip_tops*)sc.mip[uni(w.mip)].tops, sc.mip[uni(w.mip)].top};
   const int t0 = ahead + lane * kSkipSteps;
   const float bound = skip_bound(lc.end, lc.line, b, v, sc.sy, t0, t0 + kSkipSteps);
   w.bound = t0 < n ? bound : -__builtin_inff();
@@ -497,8 +516,8 @@ constexpr int kSkipReach = 2048;
 // draw above the horizon row ymin (a row the line has reached or passed) are
 // stepped over on the way.  Returns false when the line has reached the far
 // distance.
-template <bool SKIP>
-__device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const SceneDev& sc,
+template <bool SKIP, class Scene>
+__device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const Scene& sc,
                                       const LineConsts& lc, int zfar, int ymin, float* dl,
                                       int lane) {
   for (;;) {
@@ -506,11 +525,11 @@ __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const SceneDev& s
     while (w.z > (float)w.mapswitch || w.yswitch > 512.0f) {
       w.yswitch = w.yswitch * 0.5f;
       if (w.mip < sc.nmips - 1) {
-        w.mip++;
+        w.mip = uni(w.mip + 1);
         w.gridx >>= 1;
         w.gridz >>= 1;
-        w.map = sc.mip[w.mip].map;
-        w.slab = sc.mip[w.mip].slabs;
+        w.map = (g_entry*)sc.mip[w.mip].map;
+        w.slab = (g_u16*)sc.mip[w.mip].slabs;
         w.shift = sc.mip[w.mip].shift;
       }
       w.g *= 2;
@@ -536,7 +555,7 @@ __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const SceneDev& s
       for (;;) {
         if (look) dda_look_ahead(w, sc, lc, hidden, n, lane);
         const int at = max(w.ofs, 0) / kSkipSteps;  // the group of the next step
-        const uint64_t vis = uni64(__ballot(!skip_hidden(w.bound, ymin))) >> at;
+        const uint64_t vis = uni64(ballot(!skip_hidden(w.bound, ymin))) >> at;
         if (vis) {
           hidden = max((at + (int)__builtin_ctzll(vis)) * kSkipSteps - w.ofs, 0);
           break;
@@ -568,15 +587,15 @@ __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const SceneDev& s
       // term j-1 < A's term i, so i = floor((sB - sA + gA + t*gB) / (gA + gB))
       const float gr = __builtin_amdgcn_rcpf(gA + gB);
       const float e0 = (sB - sA + gA) * gr, e1 = gB * gr;
-      if (__ballot(w.q.rem < 0.0f) & 0x3f) w.q = dda_fit(w.q.s, w.g, HwRcp());
+      if (ballot(w.q.rem < 0.0f) & 0x3f) w.q = dda_fit(w.q.s, w.g, HwRcp());
       for (;;) {
         // terms the chunk may need of either kind (checked afterwards)
         const float n_steps = (float)(T + L);
         const float ex = floorf(fminf(fmaxf(e0 + e1 * n_steps, 0.0f), n_steps));
         const float nv = (xseq ? ex : n_steps - ex) + 1.0f;
         DdaTerms q{w.q.s, w.q.G, w.q.s, w.q.G, w.q.rem, w.q.rem};
-        if (__ballot(nv > w.q.rem) & 0x3f) q = dda_terms(w.q, w.g, HwRcp());
-        ok = !(__ballot(nv > q.last) & 0x3f) && dda_merge(w, c, q, T, L, e0, e1, xseq, dl, lane);
+        if (ballot(nv > w.q.rem) & 0x3f) q = dda_terms(w.q, w.g, HwRcp());
+        ok = !(ballot(nv > q.last) & 0x3f) && dda_merge(w, c, q, T, L, e0, e1, xseq, dl, lane);
         if (!SKIP || ok || T == 0) break;
         // too many binades on the way: half of it, or one chunk from here
         if (T >= 128) {
@@ -618,7 +637,10 @@ __device__ inline void dda_gather(const DdaWalk& w, DdaChunk& c, float vpx, floa
   const int vx = (voxel_x >> w.mip) & (w.gridx - 1);
   const int vz = (voxel_z >> w.mip) & (w.gridz - 1);
   c.ent = make_uint2(0u, 0u);
-  if (lane < c.L && lane >= c.first) c.ent = w.map[vx + vz * w.gridx];
+  if (lane < c.L && lane >= c.first) {
+    const v2u32 e = w.map[vx + vz * w.gridx];
+    c.ent = make_uint2(e.x, e.y);
+  }
 }
 
 // Chunks handed from the producer wavefront (DDA + pointer gather) to the
@@ -627,7 +649,7 @@ __device__ inline void dda_gather(const DdaWalk& w, DdaChunk& c, float vpx, floa
 struct ChunkRing {
   float db[3][64], dn[3][64];
   uint2 ent[3][64];
-  const uint16_t* slab[3];
+  g_u16* slab[3];
   int L[3], mip[3], shift[3], have[3];
   // written by the consumer in the round that uses the slot
   int stop[3], horizon[3];
@@ -653,7 +675,7 @@ __device__ inline void ring_get(const ChunkRing& r, int s, DdaChunk& c, int lane
   c.L = uni(r.L[s]);
   c.mip = uni(r.mip[s]);
   c.shift = uni(r.shift[s]);
-  c.slab = (const uint16_t*)uni64((uint64_t)r.slab[s]);
+  c.slab = (g_u16*)uni64((uint64_t)r.slab[s]);
   c.db = r.db[s][lane];
   c.dn = r.dn[s][lane];
   c.ent = r.ent[s][lane];
@@ -669,14 +691,20 @@ __device__ inline void ring_get(const ChunkRing& r, int s, DdaChunk& c, int lane
 // LDS arguments: bits = the line's bitmap, dl = DDA scratch, rc = run cache,
 // sweep_lds = 64 ints for the horizon sweep followed by kLineConstWords words
 // for the line's constants.
-template <bool COUNT, bool TWO = false, bool PAR_ELEMS = true, int RC = kRunCache>
-__device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_raymap& rm,
-                                        uint32_t* __restrict__ row, int32_t* __restrict__ clip,
+// Scene, Map: SceneDev and rlevox_raymap as kernel arguments or in constant
+// memory.
+template <bool COUNT, bool TWO = false, bool PAR_ELEMS = true, int RC = kRunCache, class Scene,
+          class Map>
+__device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
+                                        uint32_t* __restrict__ row_, int32_t* __restrict__ clip_,
                                         uint32_t* bits, float* dl, lds_u16* rc, int* sweep_lds,
                                         unsigned long long* counts, ChunkRing* ring = nullptr) {
   static_assert(!(COUNT && TWO), "the counting variant walks with one wavefront");
   const int lane = threadIdx.x & 63;
   const bool producer = TWO && threadIdx.x < 64;  // wavefront 0 of a two-wavefront line
+  g_u32_out* row = (g_u32_out*)row_;
+  typedef __attribute__((address_space(1))) int32_t g_i32_out;
+  g_i32_out* clip = (g_i32_out*)clip_;
   const int rs = uni(rm.rs);
   const float half = uni_f((float)(rs / 2));
   if (lane == 0 && !producer) {
@@ -727,10 +755,10 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
   if (vertical) hmul = -hmul;
   hmul = uni_f(hmul);
   const int p_add = reverse ? 1 : -2;
-  int p1x = d_f2i((float)rs * p1.x) + p_add;
-  int p1y = d_f2i((float)rs * p1.y) + p_add;
-  int p2x = d_f2i((float)rs * p2.x) - p_add;
-  int p2y = d_f2i((float)rs * p2.y) - p_add;
+  int p1x = uni(d_f2i((float)rs * p1.x)) + p_add;
+  int p1y = uni(d_f2i((float)rs * p1.y)) + p_add;
+  int p2x = uni(d_f2i((float)rs * p2.x)) - p_add;
+  int p2y = uni(d_f2i((float)rs * p2.y)) - p_add;
   p1x = min(max(p1x, 0), rs - 1);
   p1y = min(max(p1y, 0), rs - 1);
   p2x = min(max(p2x, 0), rs - 1);
@@ -774,8 +802,8 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
   const float ddx = ray_x * rm.cos_y + ray_z * rm.sin_y;
   const float ddy = ray_x * rm.sin_y - ray_z * rm.cos_y;
   float fix_xf = -1, fix_yf = -1, sign_x = -1, sign_y = -1;
-  float frac_x = vpx - (float)d_f2i(vpx);
-  float frac_y = vpz - (float)d_f2i(vpz);
+  float frac_x = vpx - (float)uni(d_f2i(vpx));
+  float frac_y = vpz - (float)uni(d_f2i(vpz));
   if (ddx >= 0) {
     fix_xf = 0;
     sign_x = 1;
@@ -806,8 +834,8 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
   wk.mip = 0;
   wk.gridx = sc.mip[0].sx;
   wk.gridz = sc.mip[0].sz;
-  wk.map = sc.mip[0].map;
-  wk.slab = sc.mip[0].slabs;
+  wk.map = (g_entry*)sc.mip[0].map;
+  wk.slab = (g_u16*)sc.mip[0].slabs;
   wk.shift = sc.mip[0].shift;
   wk.mapswitch = rm.mapswitch;
   wk.dz = 1;
@@ -842,7 +870,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
   auto chunk_step = [&](auto produce, const DdaChunk& cur, DdaChunk& nxt, bool& have_next) -> bool {
     if (ymin >= ymax) return false;
     const int L = cur.L, mip = cur.mip, shift = cur.shift;
-    const uint16_t* slab = cur.slab;
+    g_u16* slab = cur.slab;
     const uint2 ent = cur.ent;
     const uint64_t wofs = (uint64_t)ent.x << shift;  // column's slab word offset
 
@@ -861,7 +889,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     cyy *= hmul;
     const float top = pz * half + py3;
     const uint32_t slen = ent.y & 0xffffu;
-    const uint16_t* runs = slab + 2 + wofs;
+    g_u16* runs = slab + 2 + wofs;
 
     // F: projected top of the first drawn element in front of the eye.  A
     // step whose cell top is already below the horizon with pz > 0 stays
@@ -907,9 +935,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
       }
     }
 
-    // ---- run cache: the head of each candidate column, fetched now and
-    // stored to LDS after the next chunk's DDA (its latency overlaps that
-    // work).  The horizon only rises, so F > ymin now is necessary for
+    // ---- run cache: the head of each candidate column.  The horizon only rises, so F > ymin now is necessary for
     // acting; the clip-top test is monotone in ymin only for pz > 0.
     const bool cand = valid && F > ymin && !culled0;
     const uint64_t rc_base = wofs & ~(uint64_t)7;  // 16-byte aligned start
@@ -918,6 +944,10 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     const int ccap = cand ? RC - rc_delta : 0;
     static_assert(RC % 8 == 0 && RC >= 24, "the run cache is fetched in 16-byte words");
     constexpr int kWords = RC / 8;
+    // ---- next chunk's DDA, before the cache's loads go out: an LDS access
+    // waits for every load that writes LDS
+    if constexpr (decltype(produce)::value) have_next = dda_next_chunk<!COUNT>(wk, nxt, sc, *lc, zfar, ymin, dl, lane);
+
     // A wait for this wavefront's LDS reads (the last chunk's, of the cache)
     // before the loads may write it, and for the loads before it is read.
     constexpr int kWaitLds = 0xc07f, kWaitLoads = 0x0f70;  // lgkmcnt(0), vmcnt(0)
@@ -925,22 +955,12 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
       typedef __attribute__((address_space(1))) const void g_void;
       typedef __attribute__((address_space(3))) void l_void;
       __builtin_amdgcn_s_waitcnt(kWaitLds);
-      const uint16_t* src = slab + rc_base;
+      g_u16* src = slab + rc_base;
 #pragma unroll
       for (int i = 0; i < kWords; i++)
         __builtin_amdgcn_global_load_lds((g_void*)(src + 8 * i), (l_void*)(rc + 512 * i), 16, 0, 0);
     }
 
-    // ---- next chunk's DDA (the run cache loads are in flight meanwhile)
-    if constexpr (decltype(produce)::value) have_next = dda_next_chunk<!COUNT>(wk, nxt, sc, *lc, zfar, ymin, dl, lane);
-
-    // A walking wavefront waits for the cache before the gather below goes
-    // out, a drawing-only one after the span parameters.
-    if constexpr (decltype(produce)::value) __builtin_amdgcn_s_waitcnt(kWaitLoads);
-    // ---- next chunk's pointer gather: in flight during this chunk's replay
-    if constexpr (decltype(produce)::value) {
-      if (have_next) dda_gather(wk, nxt, vpx, vpz, fix_xf, fix_yf, lane);
-    }
     // first element's lower end and span parameters (Cuda_Render.h:554-660)
     int s1F = 0;
     bool drawF = false;
@@ -971,13 +991,17 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
         onedz2F /= s2r - s1rF;
       }
     }
-    if constexpr (!decltype(produce)::value) __builtin_amdgcn_s_waitcnt(kWaitLoads);
+    __builtin_amdgcn_s_waitcnt(kWaitLoads);
+    // ---- next chunk's pointer gather: in flight during this chunk's replay
+    if constexpr (decltype(produce)::value) {
+      if (have_next) dda_gather(wk, nxt, vpx, vpz, fix_xf, fix_yf, lane);
+    }
     wave_sync();  // run cache filled
     if (cand) {  // F2: projected top of the next element the loop tests
       int yg = ygF;
       for (uint32_t k = (uint32_t)kF + 1; k < slen; k++) {
         const int ci = (int)k + 2;
-        const uint32_t w = ci < ccap ? cached[ci] : runs[k];
+        const uint32_t w = column_word(ci < ccap, rc, cached.index(ci), runs + k);
         int dr = (int)(w >> 10);
         yg += (int)(w & 1023u) << mip;
         if (dr == 0) continue;
@@ -1009,7 +1033,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
       }
       const bool culled = top <= pz * (float)ymin;
       const bool act = valid && lane >= cur_step && !culled && F > ymin;
-      const uint64_t am = uni64(__ballot(act));
+      const uint64_t am = uni64(ballot(act));
       if (!COUNT && (am & (am - 1))) {
         // ---- horizon sweep: a run of acting steps applied at once.  The
         // typical step draws its first element's span from the horizon up
@@ -1028,15 +1052,15 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
         const bool true_actor = valid && lane >= cur_step && !(top <= pz * (float)M) && F > M;
         const bool simple = cand && drawF && s1F <= M && F < ymax && F2 <= F && F - ymin <= 63;
         const bool ok = spec_actor == true_actor && (!spec_actor || simple);
-        const uint64_t bad = uni64(__ballot(lane >= cur_step && !ok));
+        const uint64_t bad = uni64(ballot(lane >= cur_step && !ok));
         const int limit = uni(bad ? (int)__builtin_ctzll(bad) : 64);
-        const uint64_t acc = uni64(__ballot(spec_actor && lane < limit));
+        const uint64_t acc = uni64(ballot(spec_actor && lane < limit));
         if (acc) {
           const int last = 63 - (int)__builtin_clzll(acc);
           const int fend = uni(readlane_i(F, last));
           // rows ymin..fend (fend < ymin + 64) must all be clear
           const bool rclear = lane > fend - ymin || !lds_bit(bits, ymin + lane);
-          if (uni64(__ballot(rclear)) == ~0ull) {
+          if (uni64(ballot(rclear)) == ~0ull) {
             // row r = ymin + j belongs to the accepted step with the highest
             // start row <= j (starts are marked in LDS)
             sweep_lds[lane] = -1;
@@ -1044,7 +1068,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
             if ((acc >> lane) & 1) sweep_lds[M - ymin] = lane;
             wave_sync();
             const int mark = sweep_lds[lane];
-            const uint64_t smask = uni64(__ballot(mark >= 0));
+            const uint64_t smask = uni64(ballot(mark >= 0));
             const int nrows = fend - ymin;
             const bool mine = lane < nrows;
             const uint64_t upto = lane >= 63 ? ~0ull : ((2ull << lane) - 1ull);
@@ -1071,9 +1095,9 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
               const uint64_t wofs = (uint64_t)aofs << shift;
               const int tdelta = (int)(wofs & 7u);
               const int cw = 2 + (int)alen + tdelta + (int)u;
-              const uint32_t col = cw < RC ? rc[rc_index(a, cw)]
-                                                  : slab[2 + wofs + alen + u];
-              row[ymin + lane] = col + (depth << 16);
+              row[ymin + lane] =
+                  column_word(cw < RC, rc, rc_index(a, cw), slab + 2 + wofs + alen + u) +
+                  (depth << 16);
             }
             bits_or(bits, ymin, nrows >= 64 ? ~0ull : ((1ull << nrows) - 1ull), lane);
             wave_sync();
@@ -1088,7 +1112,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
         // no-op steps [cur_step, t): pointer loads and elements walked to the break
         const bool noop_loaded = valid && lane >= cur_step && lane < t && !culled;
         cnt.steps += (uint64_t)(t - cur_step);
-        cnt.ptr += (uint64_t)__popcll(__ballot(noop_loaded));
+        cnt.ptr += (uint64_t)__popcll(ballot(noop_loaded));
         unsigned long long e = noop_loaded ? nel : 0, r = (noop_loaded && nel) ? nel - 1 : 0;
         for (int o = 32; o > 0; o >>= 1) {
           e += __shfl_xor(e, o);
@@ -1106,8 +1130,8 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
       const uint64_t tofs = (uint64_t)(uint32_t)readlane_i((int)ent.x, t) << shift;
       const uint32_t tlf = (uint32_t)readlane_i((int)ent.y, t);
       const uint32_t tslen = tlf & 0xffffu;
-      const uint16_t* truns = slab + 2 + tofs;
-      const uint16_t* tcol = truns + tslen;
+      g_u16* truns = slab + 2 + tofs;
+      g_u16* tcol = truns + tslen;
       const bool tcached = readlane_i((int)cand, t) != 0;
       const int tdelta = (int)(tofs & 7u);
       const RcColumn tcache{rc, t, tdelta};
@@ -1178,8 +1202,10 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
         for (uint32_t base = k0; base < tslen && !stop; base += 64) {
           const uint32_t k = base + (uint32_t)lane;
           const bool in = k < tslen;
-          uint32_t w = 0;
-          if (in) w = k == 0 ? tlf >> 16 : ((int)k + 2 < tcap ? tcache[k + 2] : truns[k]);
+          const bool first = k == 0 || !in;
+          uint32_t w = column_word(first || (int)k + 2 < tcap, rc,
+                                   tcache.index(first ? 2 : (int)k + 2), truns + k);
+          w = in ? (k == 0 ? tlf >> 16 : w) : 0;
           const int edrawn = (int)(w >> 10);
           const int eskip = (int)(w & 1023u) << mip;
           const int yinc = prefix_sum_incl(eskip + (edrawn << mip), lane);
@@ -1228,7 +1254,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
           // `continue`s for it.
           const bool can_act = lane < nb && (eflags & 3) == 3 &&
                                (es2 <= ymax || ((eflags & 4) && es1 < ymax));
-          for (uint64_t act = __ballot(can_act); act != 0; act &= act - 1) {
+          for (uint64_t act = ballot(can_act); act != 0; act &= act - 1) {
             const int j = (int)__builtin_ctzll(act);
             const int f = readlane_i(eflags, j);
             if (!(f & 1) || !(f & 2)) continue;
@@ -1270,7 +1296,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
       for (uint32_t k = k0; k < tslen; k++) {
         uint32_t w;
         if (k == 0) w = tlf >> 16;
-        else w = ((int)k + 2 < tcap) ? tcache[k + 2] : truns[k];
+        else w = column_word((int)k + 2 < tcap, rc, tcache.index((int)k + 2), truns + k);
         if (COUNT) {
           cnt.elems++;
           if (k > 0) cnt.rle++;
@@ -1292,7 +1318,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
         const float pz1 = zz1 + z_add * ytop;
         if (pz1 <= 0) continue;
         const float py1 = yy1 + y_add * ytop;
-        int s2 = d_f2i(half + py1 / pz1);
+        int s2 = uni(d_f2i(half + py1 / pz1));
         if (s2 <= ymin) break;
         float zz2 = tpz, yy2 = tpy;
         if (mountain + ybot < 0) {
@@ -1302,7 +1328,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
         const float pz2 = zz2 + z_add * ybot;
         if (pz2 <= 0) continue;
         const float py2 = yy2 + y_add * ybot;
-        int s1 = d_f2i(half + py2 / pz2 - 1.0f);
+        int s1 = uni(d_f2i(half + py2 / pz2 - 1.0f));
         if (s1 >= ymax) continue;
         if (s2 >= ymax) {
           s2 = ymax;
@@ -1341,7 +1367,7 @@ __device__ inline void render_line_wave(int x, const SceneDev& sc, const rlevox_
     // ---- early end of the walk (WalkEnd): later steps lie beyond this
     // chunk's last crossing distance
     if (!done && L > 0 && !cnt.ended && wfloor < (float)ymin + (1.0f - WalkEnd::kAbs) &&
-        wend->done(readlane_f(cur.dn, L - 1), ymin, sc.mip[mip].top, sc.sy)) {
+        wend->done(readlane_f(cur.dn, L - 1), ymin, sc.mip[uni(mip)].top, sc.sy)) {
       if (COUNT) cnt.end_walk();  // the counting variant walks on to count the reference's work
       else done = true;
     }
