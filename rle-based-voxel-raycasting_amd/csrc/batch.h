@@ -8,6 +8,12 @@
 
 namespace rlevox {
 
+// Pixel rows of a tile of the batched compose and gap-fill (64 columns): a
+// persistent workgroup pays the queue, the view look-up and the staged border
+// once per tile (64 views of mixed sizes, 64x4 / 64x8 / 64x16 tiles: gap-fill
+// 1.24 / 1.06 / 0.90 ms, compose 0.91 / 0.88 / 0.75 ms).
+constexpr int kPostRows = 16;
+
 // One view of a batch, in device memory.
 struct ViewDesc {
   rlevox_raymap rm;
@@ -18,7 +24,7 @@ struct ViewDesc {
   uint16_t* colour;       // W*H output colour
   int32_t* depth;         // W*H output depth
   int64_t line_begin;     // first global line index of this view
-  int64_t tile_begin;     // first global 64x4 pixel tile of this view
+  int64_t tile_begin;     // first global pixel tile of this view
   int32_t post;           // RLEVOX_POST_* bits
   int32_t pad;
 };

@@ -115,7 +115,7 @@ __device__ inline void stage_view(const ViewDesc* __restrict__ views, int v, Vie
 __global__ __launch_bounds__(256) void k_compose_batch(BatchHeader* __restrict__ h,
                                                        const ViewDesc* __restrict__ views) {
   __shared__ ViewDesc vd;
-  __shared__ ComposeTile ct;
+  __shared__ ComposeTile<64, kPostRows> ct;
   __shared__ int64_t next[2];
   const int nv = h->nviews;
   TileWalk<DeviceAdd> walk;
@@ -133,34 +133,29 @@ __global__ __launch_bounds__(256) void k_compose_batch(BatchHeader* __restrict__
       stage_view(views, v, vd);
       staged = v;
     }
-    const int W = vd.rm.W, H = vd.rm.H;
+    const int W = vd.rm.W;
     const int local = (int)(tile - vd.tile_begin);  // < 2^18 tiles per view
     const int tiles_x = (W + 63) / 64;
     const int ty = local / tiles_x;
-    const int x0 = (local - ty * tiles_x) * 64, y0 = ty * 4;
+    const int x0 = (local - ty * tiles_x) * 64, y0 = ty * kPostRows;
     // the previous tile's reads of ct ended before this iteration's first
     // barrier
     compose_tile_stage(vd.rm, x0, y0, ct);
     __syncthreads();
-    const int px = x0 + (threadIdx.x & 63);
-    const int row = y0 + (threadIdx.x >> 6);
-    if (px < W && row < H) {
-      uint16_t c;
-      int32_t d;
-      compose_pixel(vd.rm, vd.raybuf, vd.clip, px, row, ct.col[threadIdx.x & 63],
-                    ct.row[threadIdx.x >> 6], ct.border, c, d);
-      typedef __attribute__((address_space(1))) int32_t g_i32_out;
-      g_u16_out* out = (g_u16_out*)((vd.post & RLEVOX_POST_GAPFILL) ? vd.ctmp : vd.colour);
+    typedef __attribute__((address_space(1))) int32_t g_i32_out;
+    g_u16_out* out = (g_u16_out*)((vd.post & RLEVOX_POST_GAPFILL) ? vd.ctmp : vd.colour);
+    g_i32_out* dep = (g_i32_out*)vd.depth;
+    compose_tile(vd.rm, vd.raybuf, vd.clip, x0, y0, ct, [&](int px, int row, uint16_t c, int32_t d) {
       const uint32_t i = (uint32_t)row * (uint32_t)W + (uint32_t)px;  // W, H <= 8192
       out[i] = c;
-      ((g_i32_out*)vd.depth)[i] = d;
-    }
+      dep[i] = d;
+    });
   }
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_gapfill_batch(BatchHeader* __restrict__ h,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 5))) void k_gapfill_batch(BatchHeader* __restrict__ h,
                                                        const ViewDesc* __restrict__ views) {
-  __shared__ GapTile gt;
+  __shared__ GapTile<kPostRows> gt;
   __shared__ int64_t next[2];
   const int nv = h->nviews;
   TileWalk<DeviceAdd> walk;
@@ -178,8 +173,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
     const int local = (int)(tile - vd.tile_begin);  // < 2^18 tiles per view
     const int tiles_x = (W + 63) / 64;
     const int ty = local / tiles_x;
-    gapfill_tile(W, vd.rm.H, vd.ctmp, vd.depth, vd.colour, (local - ty * tiles_x) * 64, ty * 4,
-                 gt);
+    gapfill_tile(W, vd.rm.H, vd.ctmp, vd.depth, vd.colour, (local - ty * tiles_x) * 64,
+                 ty * kPostRows, gt);
   }
 }
 
@@ -314,7 +309,7 @@ rlevox_status BatchSlot::prepare(const rlevox_view* views, int n, const rlevox_r
     d.tile_begin = tiles;
     d.post = post;
     lines += rms[i].map_line_count;
-    tiles += (int64_t)((rms[i].W + 63) / 64) * ((rms[i].H + 3) / 4);
+    tiles += (int64_t)((rms[i].W + 63) / 64) * ((rms[i].H + kPostRows - 1) / kPostRows);
     max_rs = std::max(max_rs, rms[i].rs);
     rays += (uint64_t)rms[i].W * rms[i].H;
   }

@@ -72,8 +72,12 @@ typedef __attribute__((address_space(1))) const int32_t g_i32;
 typedef __attribute__((address_space(1))) const uint16_t g_u16;
 typedef int v4i32 __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u32 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(1))) const v4i32 g_v4i32;
-typedef __attribute__((address_space(1))) const v2u32 g_v2u32;
+// Four pixels' depths or colours from any pixel on (global loads need no more
+// than the element's alignment).
+typedef int v4i32_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t v2u32_a2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef __attribute__((address_space(1))) const v4i32_a4 g_v4i32;
+typedef __attribute__((address_space(1))) const v2u32_a2 g_v2u32;
 typedef __attribute__((address_space(1))) uint16_t g_u16_out;
 typedef __attribute__((address_space(1))) uint32_t g_u32_out;
 typedef __attribute__((address_space(1))) const v2u32 g_entry;  // a pointer-map entry
@@ -488,31 +492,33 @@ __device__ inline float compose_border(const rlevox_raymap& rm) {
   return (RESX - RESY) / (RESX * 2.0f);
 }
 
-// The shared quotients of one 64x4 tile (columns x0..x0+63, rows
-// y0..y0+3): the columns by the first wavefront, the rows and the border by
-// the next two.  Call from all 256 threads; a barrier must follow before
-// the pixels read it.
+// The shared quotients of one tile: the columns by the first wavefront, the
+// rows and the border by the next two.  Call from all 256 threads; a barrier
+// must follow before the pixels read it.
+template <int COLS, int ROWS>
 struct ComposeTile {
-  ComposeCol col[64];
-  ComposeRow row[4];
+  ComposeCol col[COLS];
+  ComposeRow row[ROWS];
   float border;
 };
 
+template <int COLS, int ROWS>
 __device__ inline void compose_tile_stage(const rlevox_raymap& rm, int x0, int y0,
-                                          ComposeTile& t) {
+                                          ComposeTile<COLS, ROWS>& t) {
+  static_assert(COLS <= 64 && ROWS <= 64, "one wavefront each");
   const int i = threadIdx.x;
-  if (i < 64)
+  if (i < COLS)
     t.col[i] = compose_col(rm, x0 + i);
-  else if (i < 68)
+  else if (i >= 64 && i < 64 + ROWS)
     t.row[i - 64] = compose_row(rm, y0 + i - 64);
   else if (i == 128)
     t.border = compose_border(rm);
 }
 
-__device__ inline void compose_pixel(const rlevox_raymap& rm, const uint32_t* __restrict__ raybuf,
-                                     const int32_t* __restrict__ line_clip, int px, int prow,
-                                     ComposeCol col, ComposeRow rw, float border,
-                                     uint16_t& out_c, int32_t& out_d) {
+// The ray-buffer texel (line tr, position tc) that a pixel shows; tr < 0:
+// none.
+__device__ inline int2 compose_texel(const rlevox_raymap& rm, ComposeCol col, ComposeRow rw,
+                                     float border) {
   const float RESX = (float)rm.W, RESY = (float)rm.H;
   const int rs = rm.rs;
   const float vx = rm.vanish[0], vy = rm.vanish[1];
@@ -543,33 +549,62 @@ __device__ inline void compose_pixel(const rlevox_raymap& rm, const uint32_t* __
     tx = first ? o2 : 1.0f - o2;
   }
   ty = ty * rm.ray_ratio * 0.25f;
-  uint16_t c = RLEVOX_SKY_COLOUR;
-  int32_t d = RLEVOX_SKY_DEPTH;
-  if (isfinite(tx) && isfinite(ty)) {
-    int tc = d_f2i(floorf(tx * (float)rs));
-    int tr = d_f2i(floorf(ty * (float)(4 * rs)));
-    tc = min(max(tc, 0), rs - 1);
-    tr = min(max(tr, 0), 4 * rs - 1);
-    if (tr < rm.map_line_count) {
-      // Both loads go out together: the texel is inside the ray buffer
-      // (map_line_count x rs) for any tc, and is used only inside the
-      // line's cleared range.
-      // Read as global memory: the batch kernels take these pointers from
-      // an LDS copy of the view, where the compiler would emit flat loads
-      // and wait on both counters between them.
-      typedef __attribute__((address_space(1))) const uint64_t g_u64;
-      typedef __attribute__((address_space(1))) const uint32_t g_u32;
-      const uint32_t t = *((g_u32*)raybuf + (size_t)tr * (size_t)rs + (size_t)tc);
-      const uint64_t lcw = *(g_u64*)(line_clip + 2 * tr);  // {lo, hi}, 8-byte aligned
-      const int2 lc = make_int2((int)(uint32_t)lcw, (int)(uint32_t)(lcw >> 32));
-      // non-short-circuit test: no branch for the compiler to sink a load into
-      const bool use = (tc >= lc.x) & (tc <= lc.y) & (((t >> 16) & 0xffu) != 0xffu);
-      c = use ? (uint16_t)(t & 0xffffu) : c;
-      d = use ? (int32_t)(t >> 16) : d;
+  if (!(isfinite(tx) && isfinite(ty))) return make_int2(-1, 0);
+  int tc = d_f2i(floorf(tx * (float)rs));
+  int tr = d_f2i(floorf(ty * (float)(4 * rs)));
+  tc = min(max(tc, 0), rs - 1);
+  tr = min(max(tr, 0), 4 * rs - 1);
+  return make_int2(tr < rm.map_line_count ? tr : -1, tc);
+}
+
+// The pixels of a tile that this thread composes, written by
+// put(px, row, colour, depth).  Wavefront w of the four takes the columns
+// w*COLS/4 to (w+1)*COLS/4 - 1, 8x8 pixels at a time: the ray buffer's lines
+// run along the image's columns (upper and lower segments) or rows, so a row
+// of 64 pixels reads up to 64 lines, an 8x8 block about ten (a single frame's
+// pass: 1080p 10.0 -> 9.4 us, 4K 30.0 -> 29.5).  All loads of a thread go out
+// before the first is used.
+template <int COLS, int ROWS, class Put>
+__device__ inline void compose_tile(const rlevox_raymap& rm, const uint32_t* __restrict__ raybuf,
+                                    const int32_t* __restrict__ line_clip, int x0, int y0,
+                                    const ComposeTile<COLS, ROWS>& t, Put put) {
+  constexpr int kX = COLS / 32, kPix = kX * (ROWS / 8);
+  static_assert(COLS % 32 == 0 && ROWS % 8 == 0, "8x8 pixels per wavefront");
+  const int lane = threadIdx.x & 63;
+  const int cx = (threadIdx.x >> 6) * (COLS / 4) + (lane & 7), cy = lane >> 3;
+  // Read as global memory: the batch kernels take these pointers from an LDS
+  // copy of the view, where the compiler would emit flat loads and wait on
+  // both counters between them.
+  typedef __attribute__((address_space(1))) const uint64_t g_u64;
+  typedef __attribute__((address_space(1))) const uint32_t g_u32;
+  int2 at[kPix];
+  uint32_t tex[kPix];
+  uint64_t clip[kPix];  // {lo, hi}, 8-byte aligned
+#pragma unroll
+  for (int j = 0; j < kPix; j++)
+    at[j] = compose_texel(rm, t.col[cx + (j % kX) * 8], t.row[cy + (j / kX) * 8], t.border);
+#pragma unroll
+  for (int j = 0; j < kPix; j++) {
+    // Both loads go out together: the texel is inside the ray buffer
+    // (map_line_count x rs) for any tc, and is used only inside the line's
+    // cleared range.
+    tex[j] = 0;
+    clip[j] = 0xffffffff00000000ull;
+    if (at[j].x >= 0) {
+      tex[j] = *((g_u32*)raybuf + (size_t)at[j].x * (size_t)rm.rs + (size_t)at[j].y);
+      clip[j] = *(g_u64*)(line_clip + 2 * at[j].x);
     }
   }
-  out_c = c;
-  out_d = d;
+#pragma unroll
+  for (int j = 0; j < kPix; j++) {
+    const int px = x0 + cx + (j % kX) * 8, row = y0 + cy + (j / kX) * 8;
+    const int lo = (int)(uint32_t)clip[j], hi = (int)(uint32_t)(clip[j] >> 32);
+    const bool use = (at[j].x >= 0) & (at[j].y >= lo) & (at[j].y <= hi) &
+                     (((tex[j] >> 16) & 0xffu) != 0xffu);
+    if ((px < rm.W) & (row < rm.H))
+      put(px, row, use ? (uint16_t)(tex[j] & 0xffffu) : (uint16_t)RLEVOX_SKY_COLOUR,
+          use ? (int32_t)(tex[j] >> 16) : RLEVOX_SKY_DEPTH);
+  }
 }
 
 // Gap-fill / smoothing of one pixel (soft.frag:8-74 on integer buffers):
@@ -579,56 +614,56 @@ __device__ inline void compose_pixel(const rlevox_raymap& rm, const uint32_t* __
 __constant__ const int kRingDx[7] = {0, 9, 9, 2, -8, -10, -3};
 __constant__ const int kRingDy[7] = {10, 6, -4, -10, -7, 3, 10};
 
-__device__ inline int floor_div_pos(int a, int b) {  // b > 0
-  const int q = a / b, r = a % b;
-  return (r != 0 && r < 0) ? q - 1 : q;
-}
-
+// A pixel whose taps reach beyond the staged border (nearer than 25): dmin
+// is its ring's nearest depth, o the tap offsets of one axis.  The ten loads
+// of a tap row go out together (one after another, each waited for the last:
+// views close to the ground spent most of the pass here).
 __device__ inline uint16_t gapfill_pixel(int W, int H, g_u16* __restrict__ cin,
-                                         g_i32* __restrict__ dep, int x, int prow) {
-  const uint32_t i = (uint32_t)prow * (uint32_t)W + (uint32_t)x;
-  const uint16_t c0 = cin[i];
-  int dmin = dep[i];
-  for (int k = 0; k < 7; k++) {
-    const int xx = min(max(x + kRingDx[k], 0), W - 1);
-    const int yy = min(max(prow - kRingDy[k], 0), H - 1);
-    dmin = min(dmin, dep[(uint32_t)yy * (uint32_t)W + (uint32_t)xx]);
-  }
-  if (dmin >= RLEVOX_SKY_DEPTH) return c0;
-  const int r_q8 = 78720 / max(dmin, 1);
-  if (r_q8 < 42) return c0;
+                                         g_i32* __restrict__ dep, int x, int prow, int dmin,
+                                         const int (&o)[5], uint16_t c0) {
   int n = 1, sum = c0 & 0xff;
-  for (int a = 0; a < 5; a++) {
-    const int ox = floor_div_pos((2 * a - 5) * r_q8 + 640, 1280);
-    const int xx = min(max(x + ox, 0), W - 1);
-    for (int b = 0; b < 5; b++) {
-      const int oy = floor_div_pos((2 * b - 5) * r_q8 + 640, 1280);
-      const int yy = min(max(prow - oy, 0), H - 1);
-      const uint32_t t = (uint32_t)yy * (uint32_t)W + (uint32_t)xx;
-      const int d = dep[t];
-      if (d < RLEVOX_SKY_DEPTH && (int64_t)10 * dmin >= (int64_t)7 * d) {
-        n++;
-        sum += cin[t] & 0xff;
-      }
+  int xx[5];
+#pragma unroll
+  for (int a = 0; a < 5; a++) xx[a] = min(max(x + o[a], 0), W - 1);
+#pragma unroll 1
+  for (int b = 0; b < 5; b++) {
+    int ob = o[0];
+#pragma unroll
+    for (int i = 1; i < 5; i++) ob = b == i ? o[i] : ob;
+    const uint32_t r = (uint32_t)min(max(prow - ob, 0), H - 1) * (uint32_t)W;
+    int d[5];
+    uint32_t c[5];
+#pragma unroll
+    for (int a = 0; a < 5; a++) {
+      d[a] = dep[r + (uint32_t)xx[a]];
+      c[a] = cin[r + (uint32_t)xx[a]];
+    }
+#pragma unroll
+    for (int a = 0; a < 5; a++) {
+      const bool q = (d[a] < RLEVOX_SKY_DEPTH) & ((int64_t)10 * dmin >= (int64_t)7 * d[a]);
+      n += q ? 1 : 0;
+      sum += q ? (int)(c[a] & 0xffu) : 0;
     }
   }
   if (n > 6) return (uint16_t)((c0 & 0xff00) | ((sum + n / 2) / n));
   return c0;
 }
 
-// The same gap-fill for one 64x4 tile of a 256-thread block, with the tile
+// The same gap-fill for one 64xROWS tile of a 256-thread block, with the tile
 // and a kGapHalo-pixel border staged in LDS (coordinates clamped to the
 // image as each tap clamps them).  The ring (offsets up to 10 px) and every
 // 5x5 tap set of radius up to kGapHalo px read LDS; pixels nearer than that
 // (larger radii) read their taps from memory.  Call from all 256 threads.
 constexpr int kGapHalo = 12;
-constexpr int kGapTW = 64 + 2 * kGapHalo, kGapTH = 4 + 2 * kGapHalo;
+constexpr int kGapTW = 64 + 2 * kGapHalo;
 // One staged pixel: its depth, and its tap word (shade byte | 1 << 16 |
 // colour high byte << 24).  Summing the tap words of the qualifying taps
 // counts them in bits 16-23 and adds their shades in bits 0-15 (at most 26
 // pixels of 255), whatever the high bytes add above.
+template <int ROWS>
 struct GapTile {
-  uint2 p[kGapTH][kGapTW];
+  static constexpr int kTH = ROWS + 2 * kGapHalo;
+  uint2 p[kTH][kGapTW];
 };
 
 // The tap word of colour16 in bits 0-15 of c, or (HIGH) in bits 16-31: one
@@ -689,18 +724,20 @@ __device__ inline uint32_t gap_taps(const uint2* tp, int centre, int dmin, int d
   return acc;
 }
 
+template <int ROWS>
 __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ cin_,
                                     const int32_t* __restrict__ dep_, uint16_t* __restrict__ cout_,
-                                    int x0, int y0, GapTile& t) {
+                                    int x0, int y0, GapTile<ROWS>& t) {
+  constexpr int kGapTH = GapTile<ROWS>::kTH;
   // W, H <= 8192: pixel indices and byte offsets fit in 32 bits
   g_u16* cin = (g_u16*)cin_;
   g_i32* dep = (g_i32*)dep_;
   // uniform: a tile whose border lies inside the image needs no clamping
   const bool inner = x0 >= kGapHalo && y0 >= kGapHalo && x0 - kGapHalo + kGapTW <= W &&
                      y0 - kGapHalo + kGapTH <= H;
-  if (inner && (W & 3) == 0) {
-    // four pixels per load (x0 - kGapHalo and W are multiples of 4); every
-    // load of the thread is issued before the first store
+  if (inner) {
+    // four pixels per load; every load of the thread is issued before the
+    // first store
     constexpr int kQ = kGapTW / 4, kQuads = kQ * kGapTH, kStage = (kQuads + 255) / 256;
     static_assert(kGapTW % 4 == 0 && kGapHalo % 4 == 0, "quads must align");
     const uint32_t g0 = (uint32_t)(y0 - kGapHalo) * (uint32_t)W + (uint32_t)(x0 - kGapHalo);
@@ -754,9 +791,10 @@ __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ c
     }
   }
   __syncthreads();
-  const int lx = (threadIdx.x & 63) + kGapHalo, ly = (threadIdx.x >> 6) + kGapHalo;
-  const int x = x0 + (threadIdx.x & 63), prow = y0 + (threadIdx.x >> 6);
-  if (x < W && prow < H) {
+  const int lx = (threadIdx.x & 63) + kGapHalo, x = x0 + (threadIdx.x & 63);
+  for (int j = threadIdx.x >> 6; j < ROWS; j += 4) {  // a wavefront's rows
+    const int ly = j + kGapHalo, prow = y0 + j;
+    if (x >= W || prow >= H) break;
     const uint2 ctr = t.p[ly][lx];
     int dmin = (int)ctr.x;
     for (int k = 0; k < 7; k++) dmin = min(dmin, (int)t.p[ly - kRingDy[k]][lx + kRingDx[k]].x);
@@ -778,8 +816,8 @@ __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ c
         acc += gap_taps<4>(tp, centre, dmin, dlim);
       } else {
         const int r_q8 = div_78720(max(dmin, 1), HwRcp());  // floor(78720 / dmin)
-        // tap offsets floor(((2a-5) r + 640) / 1280); the numerators stay
-        // above -655360, so a bias of 512*1280 keeps the division unsigned
+        // tap offsets floor(((2a-5) r + 640) / 1280) with r <= 78720; a bias
+        // of 512*1280 keeps the division unsigned
         int o[5];
 #pragma unroll
         for (int a = 0; a < 5; a++)
@@ -800,7 +838,7 @@ __device__ inline void gapfill_tile(int W, int H, const uint16_t* __restrict__ c
             }
           }
         } else {
-          out = gapfill_pixel(W, H, cin, dep, x, prow);
+          out = gapfill_pixel(W, H, cin, dep, x, prow, dmin, o, out);
         }
       }
       const int n = (int)((acc >> 16) & 0xffu), sum = (int)(acc & 0xffffu);

@@ -70,46 +70,47 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(6))) void k
                                           &ring);
 }
 
+// Tiles of 32x8 pixels, one pixel per thread: a tile's quotients and its loads
+// are one chain, hidden by other workgroups (64x16 tiles of four pixels per
+// thread: 640x480 5.0 against 4.9 us, 1366x768 7.4 against 6.5).
 __global__ __launch_bounds__(256) void k_compose(rlevox_raymap rm, const uint32_t* __restrict__ raybuf,
                                                  const int32_t* __restrict__ clip,
                                                  uint16_t* __restrict__ col,
                                                  int32_t* __restrict__ dep) {
-  __shared__ ComposeTile ct;
-  const int x0 = blockIdx.x * 64, y0 = blockIdx.y * 4;
+  __shared__ ComposeTile<32, 8> ct;
+  const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 8;
   compose_tile_stage(rm, x0, y0, ct);
   __syncthreads();
-  const int px = x0 + (threadIdx.x & 63);
-  const int row = y0 + (threadIdx.x >> 6);
-  if (px >= rm.W || row >= rm.H) return;
-  uint16_t c;
-  int32_t d;
-  compose_pixel(rm, raybuf, clip, px, row, ct.col[threadIdx.x & 63], ct.row[threadIdx.x >> 6],
-                ct.border, c, d);
-  col[(size_t)row * rm.W + px] = c;
-  dep[(size_t)row * rm.W + px] = d;
+  compose_tile(rm, raybuf, clip, x0, y0, ct, [&](int px, int row, uint16_t c, int32_t d) {
+    col[(size_t)row * rm.W + px] = c;
+    dep[(size_t)row * rm.W + px] = d;
+  });
 }
 
 // Tile of block b of a grid of n tiles, gx per row: blocks are dispatched
-// round robin over the 8 XCDs, and each XCD takes groups of 8 tile rows (32
-// pixel rows), the groups dealt round robin, so the border rows that the
+// round robin over the 8 XCDs, and each XCD takes groups of 32
+// pixel rows, the groups dealt round robin, so the border rows that the
 // tiles of a group share come through the same L2 (1080p gap-fill HBM fetch
 // 99 -> 27 MB at the same speed; contiguous eighths of the image per XCD
 // fetched 15 MB but ran 2% slower, the eighths differing in work).
+template <int ROWS>
 __device__ inline int xcd_tile(int b, int n, int gx) {
-  const int G = 8 * gx, full = n / (8 * G) * (8 * G);
+  const int G = 32 / ROWS * gx, full = n / (8 * G) * (8 * G);
   if (b >= full) return b;  // the last partial round in dispatch order
   const int x = b & 7, k = b >> 3;
   return ((k / G) * 8 + x) * G + (k % G);
 }
 
+template <int ROWS>
 __global__ __launch_bounds__(256) void k_gapfill(int W, int H, const uint16_t* __restrict__ cin,
                                                  const int32_t* __restrict__ dep,
                                                  uint16_t* __restrict__ cout) {
-  __shared__ GapTile tile;
+  __shared__ GapTile<ROWS> tile;
   const int gx = (int)gridDim.x;
-  const int t = xcd_tile((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y), gx);
+  const int t = xcd_tile<ROWS>((int)(blockIdx.y * gridDim.x + blockIdx.x),
+                               (int)(gridDim.x * gridDim.y), gx);
   const int ty = t / gx;
-  gapfill_tile(W, H, cin, dep, cout, (t - ty * gx) * 64, ty * 4, tile);
+  gapfill_tile(W, H, cin, dep, cout, (t - ty * gx) * 64, ty * ROWS, tile);
 }
 
 template <int RC>
@@ -206,17 +207,35 @@ hipError_t launch_column_tops(const MipDev& m, int level, int32_t empty, int32_t
   return hipGetLastError();
 }
 
+template <int ROWS>
+static void launch_gapfill_rows(int W, int H, const uint16_t* cin, const int32_t* dep,
+                                uint16_t* cout, hipStream_t s) {
+  hipLaunchKernelGGL(k_gapfill<ROWS>, dim3((W + 63) / 64, (H + ROWS - 1) / ROWS), dim3(256), 0, s, W,
+                     H, cin, dep, cout);
+}
+
 hipError_t launch_compose(const rlevox_raymap& rm, const uint32_t* raybuf, const int32_t* clip,
                           uint16_t* col, int32_t* dep, hipStream_t s) {
-  dim3 grid((rm.W + 63) / 64, (rm.H + 3) / 4);
-  hipLaunchKernelGGL(k_compose, grid, dim3(256), 0, s, rm, raybuf, clip, col, dep);
+  hipLaunchKernelGGL(k_compose, dim3((rm.W + 31) / 32, (rm.H + 7) / 8), dim3(256), 0, s, rm, raybuf,
+                     clip, col, dep);
   return hipGetLastError();
 }
 
 hipError_t launch_gapfill(int W, int H, const uint16_t* cin, const int32_t* dep, uint16_t* cout,
                           hipStream_t s) {
-  dim3 grid((W + 63) / 64, (H + 3) / 4);
-  hipLaunchKernelGGL(k_gapfill, grid, dim3(256), 0, s, W, H, cin, dep, cout);
+  // Taller tiles stage less border per pixel (64x4: 9.6 staged pixels for
+  // each of its own, 64x8: 5.5, 64x16: 3.4) but leave fewer workgroups, and a
+  // tile's staging and taps overlap only with other tiles.  Measured in us,
+  // 4 / 8 / 16 rows: 640x480 4.8 / 5.5 / 7.7, 1280x720 9.5 / 8.9 / 9.8,
+  // 1366x768 16.5 / 17.0 / 19.4, 1920x1080 13.7 / 12.3 / 13.2, 3840x2160
+  // 52.8 / 43.6 / 42.6.
+  const int64_t pixels = (int64_t)W * H;
+  if (pixels >= 4 << 20)
+    launch_gapfill_rows<16>(W, H, cin, dep, cout, s);
+  else if (pixels >= 3 << 18)
+    launch_gapfill_rows<8>(W, H, cin, dep, cout, s);
+  else
+    launch_gapfill_rows<4>(W, H, cin, dep, cout, s);
   return hipGetLastError();
 }
 

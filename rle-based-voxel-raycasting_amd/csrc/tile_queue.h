@@ -16,7 +16,8 @@
 // the back requests n-1, n-2, ..., and every chunk goes once.  Each queue
 // word has a 256-byte line of its own: requests to one address are served
 // one at a time by the memory (a C4 batch's 710400 single-tile requests
-// to one line took 4.5 ms).
+// to one line took 4.5 ms).  The tiles are 64x16 pixels, so a stripe is 256
+// of them and a chunk one.
 #pragma once
 
 #include <stdint.h>
@@ -24,10 +25,10 @@
 namespace rlevox {
 
 #ifndef RLEVOX_TILE_STRIPE
-#define RLEVOX_TILE_STRIPE 1024
+#define RLEVOX_TILE_STRIPE 256
 #endif
 #ifndef RLEVOX_TILE_CHUNK
-#define RLEVOX_TILE_CHUNK 4
+#define RLEVOX_TILE_CHUNK 1
 #endif
 constexpr int kTileStripe = RLEVOX_TILE_STRIPE;
 constexpr int kTileChunk = RLEVOX_TILE_CHUNK;
