@@ -17,6 +17,7 @@
 #include "walk_end.h"
 #include "walk_skip.h"
 #include "recip_div.h"
+#include "exact_div.h"
 
 namespace rlevox {
 

@@ -197,6 +197,54 @@ __device__ inline uint32_t column_word(bool cached, const lds_u16* rc, int index
   return w;
 }
 
+// Sets the bitmap bits of rows [from, to), to <= from + 64: lane l < 3 ORs
+// word l of the range.
+__device__ inline void bits_set_range(uint32_t* bits, int from, int to, int lane) {
+  const int w = (from >> 5) + lane;
+  const int lo = max(from - 32 * w, 0), hi = min(to - 32 * w, 32);
+  if (lane < 3 && lo < hi) atomicOr(&bits[w], (~0u << lo) & (~0u >> (32 - hi)));
+}
+
+// The n-th of a span's per-pixel increments from (uz, oz) on
+// (Cuda_Render.h:687): n additions each, the last ones of a multiple of four
+// without a test between them.
+__device__ inline void span_steps(float& uz, float& oz, float u2dz, float onedz2, int n) {
+  if (n & 1) {
+    uz += u2dz;
+    oz += onedz2;
+  }
+  if (n & 2) {
+    uz += u2dz;
+    oz += onedz2;
+    uz += u2dz;
+    oz += onedz2;
+  }
+  for (n >>= 2; n > 0; n--) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      uz += u2dz;
+      oz += onedz2;
+    }
+  }
+}
+
+// A pixel's colour index and depth (Cuda_Render.h:690-723) from its u/z and
+// 1/z.  tlo and thi are integers below 2^24, so the index needs no clamp.
+__device__ inline void span_texel(float uz, float oz, float tlo, float thi, uint32_t& u,
+                                  uint32_t& depth) {
+  float z, v;
+  const bool safe = div_safe(oz) & div_dividend_safe(uz);
+  if (ballot(!safe) == 0) {  // both quotients from one reciprocal
+    z = recip_exact(oz, __builtin_amdgcn_rcpf(oz));
+    v = div_exact(uz, oz, z);
+  } else {
+    z = 1.0f / oz;
+    v = uz / oz;
+  }
+  u = (uint32_t)d_f2i(fminf(fmaxf(v, tlo), thi));
+  depth = (uint32_t)d_f2i(z) & 0xfffeu;
+}
+
 // Draws pixels [y0, s2) of one span (uniform arguments; Cuda_Render.h:
 // 678-733).  Pixel y0+k has had k per-pixel increments.
 __device__ inline int draw_span(int y0, int s2, float uzb, float ozb, float u2dz, float onedz2,
@@ -206,17 +254,12 @@ __device__ inline int draw_span(int y0, int s2, float uzb, float ozb, float u2dz
   int drawn = 0;
   for (int base = y0; base < s2; base += 64) {
     float uz = uzb, oz = ozb;
-    const int adds = min(lane, s2 - 1 - base);
-    for (int i = 0; i < adds; i++) {
-      uz += u2dz;
-      oz += onedz2;
-    }
+    span_steps(uz, oz, u2dz, onedz2, max(min(lane, s2 - 1 - base), 0));
     const int y = base + lane;
     const bool draw = y < s2 && !lds_bit(bits, y);
     if (draw) {
-      const float fu = fminf(fmaxf(uz / oz, tlo), thi);
-      const uint32_t u = (uint32_t)d_f2i(fu);
-      const uint32_t depth = (uint32_t)d_f2i(1.0f / oz) & 0xfffeu;
+      uint32_t u, depth;
+      span_texel(uz, oz, tlo, thi, u, depth);
       const int cw = cofs + (int)u;
       row[y] = column_word(cw < ccap, cached.rc, cached.index(cw), colours + u) + (depth << 16);
     }
@@ -267,13 +310,9 @@ __device__ inline int span_draw(const SpanWindow& w, int s1, int e2, float uzb, 
                      bits, lane);
   if ((w.m >> lane) & 1) {
     float uz = uzb, oz = ozb;
-    for (int i = w.y0 - s1; i < lane; i++) {
-      uz += u2dz;
-      oz += onedz2;
-    }
-    const float fu = fminf(fmaxf(uz / oz, tlo), thi);
-    const uint32_t u = (uint32_t)d_f2i(fu);
-    const uint32_t depth = (uint32_t)d_f2i(1.0f / oz) & 0xfffeu;
+    span_steps(uz, oz, u2dz, onedz2, lane - (w.y0 - s1));  // row y0 or later
+    uint32_t u, depth;
+    span_texel(uz, oz, tlo, thi, u, depth);
     const int cw = cofs + (int)u;
     row[s1 + lane] =
         column_word(cw < ccap, cached.rc, cached.index(cw), colours + u) + (depth << 16);
@@ -976,19 +1015,48 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
       if (pz2 > 0) {
         drawF = true;
         const float py2 = yy2 + y_add * ybotF;
-        s1F = d_f2i(half + py2 / pz2 - 1.0f);
         const float pz1r = pz + z_add * ytopF;
         const float py1r = py3 + y_add * ytopF;
         const float pz2r = pz + z_add * ybotF;
         const float py2r = py3 + y_add * ybotF;
-        const float s2r = half + py1r / pz1r;
-        s1rF = half + py2r / pz2r;
-        u1zF = texF / pz2r;
-        u2dzF = (float)textureF / pz1r - u1zF;
-        onez1F = 1.0f / pz2r;
-        onedz2F = 1.0f / pz1r - onez1F;
-        u2dzF /= s2r - s1rF;
-        onedz2F /= s2r - s1rF;
+        // The quotients by pz1r, pz2r and the span's length share their
+        // divisors' reciprocals (exact_div.h): 43 instructions in place of 99
+        // for the nine.  |py| below 2^-60 is fine, next to half >= 8.
+        const bool safe = div_safe(pz1r) & div_safe(pz2r) &
+                          (fmaxf(fabsf(py1r), fabsf(py2r)) < 1152921504606846976.0f);
+        if (ballot(!safe) == 0) {
+          onez1F = recip_exact(pz2r, __builtin_amdgcn_rcpf(pz2r));
+          const float onez2 = recip_exact(pz1r, __builtin_amdgcn_rcpf(pz1r));
+          const float q2 = div_exact(py2r, pz2r, onez1F);
+          const float len = (half + div_exact(py1r, pz1r, onez2)) - (half + q2);
+          s1rF = half + q2;
+          u1zF = div_exact(texF, pz2r, onez1F);
+          u2dzF = div_exact((float)textureF, pz1r, onez2) - u1zF;
+          onedz2F = onez2 - onez1F;
+          // the bottom edge itself, unless the near-edge correction moved it
+          s1F = d_f2i(half + q2 - 1.0f);
+          const bool moved = mountain + ybotF < 0;
+          if (ballot(moved) != 0 && moved) s1F = d_f2i(half + py2 / pz2 - 1.0f);
+          const bool safe_len = div_safe(len) & div_dividend_safe(u2dzF) & div_dividend_safe(onedz2F);
+          if (ballot(!safe_len) == 0) {
+            const float r = recip_exact(len, __builtin_amdgcn_rcpf(len));
+            u2dzF = div_exact(u2dzF, len, r);
+            onedz2F = div_exact(onedz2F, len, r);
+          } else {
+            u2dzF /= len;
+            onedz2F /= len;
+          }
+        } else {
+          s1F = d_f2i(half + py2 / pz2 - 1.0f);
+          const float s2r = half + py1r / pz1r;
+          s1rF = half + py2r / pz2r;
+          u1zF = texF / pz2r;
+          u2dzF = (float)textureF / pz1r - u1zF;
+          onez1F = 1.0f / pz2r;
+          onedz2F = 1.0f / pz1r - onez1F;
+          u2dzF /= s2r - s1rF;
+          onedz2F /= s2r - s1rF;
+        }
       }
     }
     __builtin_amdgcn_s_waitcnt(kWaitLoads);
@@ -1085,21 +1153,17 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
               const int y0 = ymin + srow;
               const float mult = (float)(y0 + 1) - s1r;
               float uz = u1z + u2dz * mult, oz = onez1 + onedz2 * mult;
-              for (int i = srow; i < lane; i++) {
-                uz += u2dz;
-                oz += onedz2;
-              }
-              const float fu = fminf(fmaxf(uz / oz, tlo), thi);
-              const uint32_t u = (uint32_t)d_f2i(fu);
-              const uint32_t depth = (uint32_t)d_f2i(1.0f / oz) & 0xfffeu;
+              span_steps(uz, oz, u2dz, onedz2, lane - srow);
+              uint32_t u, depth;
+              span_texel(uz, oz, tlo, thi, u, depth);
               const uint64_t wofs = (uint64_t)aofs << shift;
-              const int tdelta = (int)(wofs & 7u);
+              const int tdelta = (int)((aofs << shift) & 7u);
               const int cw = 2 + (int)alen + tdelta + (int)u;
               row[ymin + lane] =
                   column_word(cw < RC, rc, rc_index(a, cw), slab + 2 + wofs + alen + u) +
                   (depth << 16);
             }
-            bits_or(bits, ymin, nrows >= 64 ? ~0ull : ((1ull << nrows) - 1ull), lane);
+            bits_set_range(bits, ymin, fend, lane);
             wave_sync();
             ymin = fend;
             cur_step = limit;
