@@ -177,23 +177,23 @@ typedef struct {
                               consecutive DDA steps); 16, 32 or 64 = one lane
                               per line */
   int32_t waves_per_block; /* 1..4; with lines_per_wave 1: 1 = one wavefront
-                              both walks and draws a line, 2..4 = two
+                              both walks and draws a line, 2 or 4 = two
                               wavefronts per line, one walking the DDA ahead
-                              of the one drawing, 0 = two when the frame
-                              has at most 14 lines per compute unit, else
-                              one (single renders: the batched kernels keep
-                              one wavefront per line, which uses a full GPU
-                              better) */
+                              of the one drawing, 3 = three, with one between
+                              them that projects and fetches columns, 0 = by
+                              the frame: one when it is wider than 2560,
+                              three up to 1792 lines, else two (single
+                              renders: the batched kernels keep one wavefront
+                              per line, which uses a full GPU better) */
   int32_t persistent_waves; /* wavefronts per CU of the persistent batch kernel
                                (0 = default 16, else 4..32) */
   int32_t order;           /* 0 = view order, 1 = longest views first */
   int32_t run_cache;       /* LDS run-cache words per candidate column of the
                               wavefront-per-line kernels (24, 40 or 56; 0 =
-                              40 with two wavefronts per line, 56 with one):
-                              deeper holds more of a column's runs and
+                              24): deeper holds more of a column's runs and
                               colours in LDS, shallower loads less per
                               column */
-  int32_t batch_run_cache; /* the same for the persistent batch kernel (0 = 40) */
+  int32_t batch_run_cache; /* the same for the persistent batch kernel (0 = 24) */
   int32_t batch_par;       /* element replay of the persistent batch kernel:
                               0 = chosen by the scenes' runs per column
                               (lane-parallel above 7), 1 = element by

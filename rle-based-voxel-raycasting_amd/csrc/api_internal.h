@@ -89,7 +89,7 @@ struct BatchSlot {
   int nviews = 0;
   int waves = kWavesPerCU;        // persistent wavefronts per CU of this batch
   bool par_elems = false;         // raycast with the lane-parallel element replay
-  int run_cache = 40;             // LDS run-cache words of the raycast
+  int run_cache = 24;             // LDS run-cache words of the raycast
   int graph_waves = 0;            // the values the captured graph was made with
   bool graph_par = false;
   int graph_rc = 0;
@@ -132,7 +132,7 @@ struct rlevox_ctx {
     return it == tuned.end() ? tuning : it->second;
   }
   // Widest ray-buffer line (screen width) up to which the automatic choice
-  // walks each line with two wavefronts, one on the DDA and one drawing.
+  // walks each line with several wavefronts, one on the DDA and one drawing.
   // Measured over the 100-pose flythrough of the 4096^2 terrain (mean
   // raycast ms, two wavefronts / one with a 56-word run cache): 640x480
   // 0.091 / 0.122, 1280x720 0.100 / 0.128, 1920x1080 0.118 / 0.141,
@@ -140,13 +140,22 @@ struct rlevox_ctx {
   // line count, up to 4096 and more lines), 3200x1800 0.210 / 0.186,
   // 3840x2160 0.251 / 0.229.
   static constexpr int kTwoWaveMaxWidth = 2560;
-  // 1 selects the wavefront-per-line kernel, 2 its two-wavefront form;
+  // Lines up to which a line of that width is walked by three wavefronts: the
+  // lines whose LDS (21 KB each) the 256 compute units hold at once.  With
+  // them all resident a frame takes as long as its longest line, which three
+  // wavefronts walk faster; beyond, lines wait for LDS (us per frame, three
+  // / two: 320x240, 441 lines, 83 / 91; 640x480, 882-1125 lines, 79 / 88;
+  // 1366x768, 1532-1654 lines, 98 / 99; 1280x720, 1626-1891 lines, 88 / 94;
+  // 1920x1080, 2048-3050 lines, 170 / 132).
+  static constexpr int kThreeWaveMaxLines = 1792;
+  // 1 selects the wavefront-per-line kernel, 2 and 3 its forms with more;
   // otherwise lanes per block (16 or more), halved until the block's
   // per-lane bitmaps (ceil(rs/32) words each) fit the workgroup's LDS.
   int tuning_block(const rlevox_tuning& t, int lines, int rs) const {
     if (t.lines_per_wave == 1) {
-      if (t.waves_per_block == 0) return rs <= kTwoWaveMaxWidth ? 2 : 1;
-      return t.waves_per_block >= 2 ? 2 : 1;
+      if (t.waves_per_block == 0)
+        return rs > kTwoWaveMaxWidth ? 1 : lines > kThreeWaveMaxLines ? 2 : 3;
+      return t.waves_per_block == 4 ? 2 : t.waves_per_block;
     }
     int block = t.lines_per_wave * t.waves_per_block;
     const size_t lane_bytes = (size_t)rlevox::bitmap_words(rs) * sizeof(uint32_t);

@@ -705,7 +705,7 @@ __device__ inline uint32_t gap_taps(const uint2* tp, int centre, int dmin, int d
     w[1] = 4;
   } else {
     const bool c2 = dmin > kGap2, c4 = dmin <= kGap3;  // 2x2, 4x4 lanes
-    w[N - 3] = c2 | c4 ? 1 : 2;  // -1
+    w[N - 3] = (c2 | c4) ? 1 : 2;  // -1
     w[N - 2] = c2 ? 4 : 2;       // 0
     w[N - 1] = c2 ? 0 : 1;       // 1
     if (N == 4) w[0] = c4 ? 1 : 0;

@@ -44,7 +44,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
   extern __shared__ uint32_t lds[];
   if ((int)blockIdx.x >= rm.map_line_count) return;
   const int x = rm.map_line_count - 1 - (int)blockIdx.x;  // last line first
-  render_line_wave<COUNT, false, true, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
+  render_line_wave<COUNT, 1, true, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
                                            clip + 2 * x, lds, dda,
                                            (lds_u16*)rcache, sweep, counts);
 }
@@ -64,10 +64,31 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(6))) void k
   extern __shared__ uint32_t lds[];
   if ((int)blockIdx.x >= rm.map_line_count) return;
   const int x = rm.map_line_count - 1 - (int)blockIdx.x;  // last line first
-  render_line_wave<false, true, true, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
+  render_line_wave<false, 2, true, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
                                           clip + 2 * x, lds, dda,
                                           (lds_u16*)rcache, sweep, nullptr,
                                           &ring);
+}
+
+// Three wavefronts per ray line: one walks, one projects and fetches the
+// columns, one draws.  A frame of few lines takes as long as its longest one
+// (320x240: 45 chunks at 3.7 K cycles), and that line's round was the longer
+// of its walk (2.6 K cycles) and its step (1.4 K to prepare, 1.4 K to draw).
+template <int RC>
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(5))) void k_raycast_wave3(SceneDev sc, rlevox_raymap rm,
+                                                       uint32_t* __restrict__ raybuf,
+                                                       int32_t* __restrict__ clip) {
+  __shared__ uint4 rcache[kPrepSlots * 64 * RC / 8];
+  __shared__ int sweep[64 + kLineConstWords];
+  __shared__ __align__(16) float dda[kDdaLds];
+  __shared__ LineRings rings;
+  extern __shared__ uint32_t lds[];
+  if ((int)blockIdx.x >= rm.map_line_count) return;
+  const int x = rm.map_line_count - 1 - (int)blockIdx.x;  // last line first
+  render_line_wave<false, 3, true, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
+                                          clip + 2 * x, lds, dda,
+                                          (lds_u16*)rcache, sweep, nullptr,
+                                          nullptr, &rings);
 }
 
 // Tiles of 32x8 pixels, one pixel per thread: a tile's quotients and its loads
@@ -114,10 +135,13 @@ __global__ __launch_bounds__(256) void k_gapfill(int W, int H, const uint16_t* _
 }
 
 template <int RC>
-static void launch_wave(const SceneDev& sc, const rlevox_raymap& rm, uint32_t* raybuf,
-                        int32_t* clip, bool two, hipStream_t s) {
+static void launch_waves(const SceneDev& sc, const rlevox_raymap& rm, uint32_t* raybuf,
+                        int32_t* clip, int waves, hipStream_t s) {
   const size_t lds = (size_t)bitmap_words(rm.rs) * sizeof(uint32_t);
-  if (two)
+  if (waves == 3)
+    hipLaunchKernelGGL(k_raycast_wave3<RC>, dim3(rm.map_line_count), dim3(192), lds, s, sc, rm,
+                       raybuf, clip);
+  else if (waves == 2)
     hipLaunchKernelGGL(k_raycast_wave2<RC>, dim3(rm.map_line_count), dim3(128), lds, s, sc, rm,
                        raybuf, clip);
   else
@@ -130,22 +154,22 @@ hipError_t launch_raycast_plain(const SceneDev& sc, const rlevox_raymap& rm, uin
                                 unsigned long long* counts) {
   const int lines = rm.map_line_count;
   if (lines <= 0) return hipSuccess;
-  if (block == 1 || block == 2) {  // wavefront kernels
-    // Default depth: 40 words with two wavefronts per line (1080p
-    // flythrough: 0.1504 ms vs 0.1509 / 0.1514 with 24 / 56), 56 with one,
-    // where frames have many long lines (4K flythrough 0.267 vs 0.272 ms,
-    // 4K grazing views of the 16384^2 terrain 8.03 vs 8.10 ms).
-    if (run_cache == 0) run_cache = block == 2 ? kRunCache : 56;
+  if (block >= 1 && block <= 3) {  // wavefront kernels
+    // Default depth 24: with the cache loaded straight into LDS the deeper
+    // ones save no time and hold LDS (us with 24 / 40 / 56: four 1080p
+    // frames 572 / 574 / -, four at 4K 1120 / 1125 / 1127, four grazing ones
+    // 969 / 971 / 976; 640x480 with three wavefronts 325 / 327 / -).
+    if (run_cache == 0) run_cache = 24;
     if (counts) {  // counting walks with one wavefront and the default run cache
       const size_t lds = (size_t)bitmap_words(rm.rs) * sizeof(uint32_t);
       hipLaunchKernelGGL((k_raycast_wave<true, kRunCache>), dim3(lines), dim3(64), lds, s, sc, rm,
                          raybuf, clip, counts);
     } else if (run_cache == 24) {
-      launch_wave<24>(sc, rm, raybuf, clip, block == 2, s);
+      launch_waves<24>(sc, rm, raybuf, clip, block, s);
     } else if (run_cache == 56) {
-      launch_wave<56>(sc, rm, raybuf, clip, block == 2, s);
+      launch_waves<56>(sc, rm, raybuf, clip, block, s);
     } else {
-      launch_wave<kRunCache>(sc, rm, raybuf, clip, block == 2, s);
+      launch_waves<kRunCache>(sc, rm, raybuf, clip, block, s);
     }
     return hipGetLastError();
   }

@@ -37,6 +37,9 @@
 //     gathers (1-2), the other projects, caches and draws (3-7); chunks pass
 //     between them through a three-slot LDS ring with one workgroup barrier
 //     per chunk.
+//  9. Three-wavefront form (k_raycast_wave3): one wavefront walks (1-2), one
+//     prepares (3-4), one draws (5-7), each as far ahead of the next as two
+//     rings in LDS allow.
 #pragma once
 
 #include <type_traits>
@@ -80,8 +83,8 @@ __device__ inline void wave_sync() {
 
 // Slab words cached per step (from the 16-byte boundary at or below the
 // column header): covers header, elements and colours of typical columns.
-// The default depth; the wavefront-per-line kernels are also built for 24
-// and 56 words (a tuning choice).
+// The counting walk's depth; the other kernels are built for 24, 40 and 56
+// words (a tuning choice).
 constexpr int kRunCache = 40;
 // The cache holds 16-byte words of 8 slab words, word i of all 64 lanes'
 // columns side by side: the layout in which the loads write LDS themselves
@@ -720,33 +723,150 @@ __device__ inline void ring_get(const ChunkRing& r, int s, DdaChunk& c, int lane
   c.ent = r.ent[s][lane];
 }
 
-// TWO: the line is walked by a 128-thread block, wavefront 0 producing the
+// A step's stateless projection (Cuda_Render.h:444-466).
+struct StepProj {
+  float pz, py3, czz, cyy, top;
+};
+
+// A chunk as the replay needs it: per lane the step's distances and column,
+// its first drawn element in front of the eye (F: projected top) and the top
+// F2 of the next element the loop tests.
+struct DdaPrepared {
+  int L, mip, shift;
+  g_u16* slab;
+  float db, dn;
+  uint2 ent;
+  int F, F2, kF, ygF, textureF, s1F;
+  bool cand, drawF;
+  float texF, s1rF, u1zF, u2dzF, onez1F, onedz2F;
+  uint32_t nel;  // elements looked at (counted by the counting walk only)
+};
+constexpr int kPreparedWords = 16;  // per lane: all but L, mip, shift, slab, nel
+
+// A three-wavefront line's hand-offs: walked chunks through one ring,
+// prepared ones (and their run caches) through another.  A wavefront waits
+// only where a slot is missing, on a counter in LDS: a chunk without
+// candidates is prepared in a third of the time of one with, a walk over a
+// hidden stretch takes twice a plain one, and a barrier per chunk would
+// charge every round the longest of the three.  The waits sleep 256 or 512
+// cycles a turn: polling every 64 cost the other lines' wavefronts issue slots
+// (1366x768 400 us against 394).  More walked chunks ahead are walked with an
+// older horizon and hold LDS (3 / 4 / 6 slots: 1280x720 727 / 715 / 718 us).
+constexpr int kWalkSlots = 4, kPrepSlots = 2;
+struct LineRings {
+  float db[kWalkSlots][64], dn[kWalkSlots][64];
+  uint2 ent[kWalkSlots][64];
+  uint32_t prep[kPrepSlots][kPreparedWords][64];
+  g_u16 *slab[kWalkSlots], *pslab[kPrepSlots];
+  int L[kWalkSlots], mip[kWalkSlots], shift[kWalkSlots];
+  int pL[kPrepSlots], pmip[kPrepSlots], pshift[kPrepSlots];
+  // chunks complete in either ring so far, and the line's chunks (INT32_MAX
+  // until the walk, the preparation has ended)
+  int walked, walk_total, prepared, prep_total;
+  int taken;  // walked chunks read from their slots
+  // prepared chunks replayed, whether the line has ended, its horizon
+  int replayed, stop, horizon;
+  LineConsts lc;  // the walker's
+};
+
+// The counters above, each written by one wavefront and read by others.  A
+// wavefront's LDS instructions execute in program order, so one that reads a
+// counter finds what its writer had written or read in the rings before it;
+// wave_sync keeps the compiler to that order.  All wavefronts of a block are
+// resident, and each wait ends with another's next chunk or its end.
+__device__ inline int ring_read(const int& v) {
+  return uni(__hip_atomic_load(&v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+__device__ inline void ring_write(int& at, int v, int lane) {
+  wave_sync();
+  if (lane == 0) __hip_atomic_store(&at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ inline void prep_put(LineRings& r, int s, const DdaPrepared& p, int lane) {
+  auto put = [&](int i, uint32_t v) { r.prep[s][i][lane] = v; };
+  auto putf = [&](int i, float v) { put(i, __float_as_uint(v)); };
+  put(0, p.ent.x);
+  put(1, p.ent.y);
+  putf(2, p.db);
+  putf(3, p.dn);
+  put(4, (uint32_t)p.F);
+  put(5, (uint32_t)p.F2);
+  put(6, (uint32_t)p.kF);
+  put(7, (uint32_t)p.ygF);
+  put(8, (uint32_t)p.textureF | (p.cand ? 1u << 30 : 0u) | (p.drawF ? 1u << 31 : 0u));
+  put(9, (uint32_t)p.s1F);
+  putf(10, p.texF);
+  putf(11, p.s1rF);
+  putf(12, p.u1zF);
+  putf(13, p.u2dzF);
+  putf(14, p.onez1F);
+  putf(15, p.onedz2F);
+  if (lane == 0) {
+    r.pslab[s] = p.slab;
+    r.pL[s] = p.L;
+    r.pmip[s] = p.mip;
+    r.pshift[s] = p.shift;
+  }
+}
+
+__device__ inline void prep_get(const LineRings& r, int s, DdaPrepared& p, int lane) {
+  auto get = [&](int i) { return r.prep[s][i][lane]; };
+  auto getf = [&](int i) { return __uint_as_float(get(i)); };
+  p.L = uni(r.pL[s]);
+  p.mip = uni(r.pmip[s]);
+  p.shift = uni(r.pshift[s]);
+  p.slab = (g_u16*)uni64((uint64_t)r.pslab[s]);
+  p.ent = make_uint2(get(0), get(1));
+  p.db = getf(2);
+  p.dn = getf(3);
+  p.F = (int)get(4);
+  p.F2 = (int)get(5);
+  p.kF = (int)get(6);
+  p.ygF = (int)get(7);
+  p.cand = (get(8) >> 30) & 1u;  // textureF: 0 to 2^24
+  p.drawF = get(8) >> 31;
+  p.textureF = (int)(get(8) & 0x3fffffffu);
+  p.s1F = (int)get(9);
+  p.texF = getf(10);
+  p.s1rF = getf(11);
+  p.u1zF = getf(12);
+  p.u2dzF = getf(13);
+  p.onez1F = getf(14);
+  p.onedz2F = getf(15);
+}
+
+// WAVES: wavefronts of the line's block.  Of two, wavefront 0 produces the
 // DDA chunks (and their pointer gathers) two chunks ahead of wavefront 1,
-// which consumes them; the two halves of the work overlap.  Otherwise one
-// wavefront does both, software-pipelined.  PAR_ELEMS: the ordered replay
+// which consumes them; the two halves of the work overlap.  Of three, the
+// second prepares chunks for the third (LineRings).  One wavefront does both,
+// software-pipelined.  PAR_ELEMS: the ordered replay
 // precomputes a column's remaining elements across the lanes (pays where
 // steps often show several elements, as in grazing views of caved terrain;
 // the persistent batch kernel leaves it off, where its registers spill).
-// LDS arguments: bits = the line's bitmap, dl = DDA scratch, rc = run cache,
+// LDS arguments (rc holds kPrepSlots caches for three wavefronts): bits = the line's bitmap, dl = DDA scratch, rc = run cache,
 // sweep_lds = 64 ints for the horizon sweep followed by kLineConstWords words
 // for the line's constants.
 // Scene, Map: SceneDev and rlevox_raymap as kernel arguments or in constant
 // memory.
-template <bool COUNT, bool TWO = false, bool PAR_ELEMS = true, int RC = kRunCache, class Scene,
+template <bool COUNT, int WAVES = 1, bool PAR_ELEMS = true, int RC = kRunCache, class Scene,
           class Map>
 __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
                                         uint32_t* __restrict__ row_, int32_t* __restrict__ clip_,
                                         uint32_t* bits, float* dl, lds_u16* rc, int* sweep_lds,
-                                        unsigned long long* counts, ChunkRing* ring = nullptr) {
-  static_assert(!(COUNT && TWO), "the counting variant walks with one wavefront");
+                                        unsigned long long* counts, ChunkRing* ring = nullptr,
+                                        LineRings* rings = nullptr) {
+  static_assert(!(COUNT && WAVES > 1), "the counting variant walks with one wavefront");
+  constexpr bool TWO = WAVES == 2;
   const int lane = threadIdx.x & 63;
-  const bool producer = TWO && threadIdx.x < 64;  // wavefront 0 of a two-wavefront line
+  // wavefront 0 of several walks; the last one draws
+  const bool producer = WAVES > 1 && threadIdx.x < 64;
+  const bool drawer = WAVES == 1 || (int)threadIdx.x >= 64 * (WAVES - 1);
   g_u32_out* row = (g_u32_out*)row_;
   typedef __attribute__((address_space(1))) int32_t g_i32_out;
   g_i32_out* clip = (g_i32_out*)clip_;
   const int rs = uni(rm.rs);
   const float half = uni_f((float)(rs / 2));
-  if (lane == 0 && !producer) {
+  if (lane == 0 && drawer) {
     clip[0] = 0;
     clip[1] = -1;
   }
@@ -823,7 +943,7 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
   if (ymin >= ymax) return;
 
   // ---- clear the range and the bitmap (Cuda_Render.h:255-264), coalesced
-  if (!producer) {
+  if (drawer) {
     for (int n = ymin + lane; n <= ymax; n += 64) row[n] = RLEVOX_CLEAR_TEXEL;
     const int words = bitmap_words(rs);
     for (int w = lane; w < words; w += 64) bits[w] = 0;
@@ -890,9 +1010,10 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
   // the line's constants, in LDS behind the sweep marks (the producer of a
   // two-wavefront line has its own)
   LineConsts* lc = reinterpret_cast<LineConsts*>(sweep_lds + 64);
-  if (producer) lc = &ring->lc;
+  if (TWO && producer) lc = &ring->lc;
+  if (WAVES == 3 && producer) lc = &rings->lc;
   const WalkEnd* wend = &lc->end;
-  if (lane == 0) {
+  if (lane == 0 && (producer || drawer)) {
     lc->end.init(cos_x, sin_x, hmul, ray_x, ray_z, vertical, mountain, half);
     lc->line.init(ddx, ddy, vpx, vpz);
   }
@@ -906,8 +1027,24 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
   // computed past the end of the line is simply dropped.  The step's code
   // appears once (unrolled over two register sets it took 40 KB of the 64 KB
   // instruction cache that two compute units share).
-  auto chunk_step = [&](auto produce, const DdaChunk& cur, DdaChunk& nxt, bool& have_next) -> bool {
-    if (ymin >= ymax) return false;
+  auto project = [&](float db, float dn) {
+    const float ddelta = dn - db;
+    const float vs_x = ray_x * db;
+    const float vs_z = ray_z * db;
+    const float corr_x = ray_x * ddelta;
+    const float corr_z = ray_z * ddelta;
+    StepProj p;
+    p.pz = cos_x * vs_z + sin_x * mountain;
+    p.py3 = vertical ? cos_x * mountain - sin_x * vs_z : vs_x;
+    p.py3 *= hmul;
+    p.czz = cos_x * corr_z;
+    p.cyy = vertical ? -sin_x * corr_z : corr_x;
+    p.cyy *= hmul;
+    p.top = p.pz * half + p.py3;
+    return p;
+  };
+  auto prepare = [&](auto produce, const DdaChunk& cur, DdaChunk& nxt, bool& have_next,
+                     lds_u16* rc, DdaPrepared& out) {
     const int L = cur.L, mip = cur.mip, shift = cur.shift;
     g_u16* slab = cur.slab;
     const uint2 ent = cur.ent;
@@ -915,18 +1052,8 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
 
     // ---- per-lane stateless projection (Cuda_Render.h:444-466)
     const bool valid = lane < L;
-    const float ddelta = cur.dn - cur.db;
-    const float vs_x = ray_x * cur.db;
-    const float vs_z = ray_z * cur.db;
-    const float corr_x = ray_x * ddelta;
-    const float corr_z = ray_z * ddelta;
-    const float pz = cos_x * vs_z + sin_x * mountain;
-    float py3 = vertical ? cos_x * mountain - sin_x * vs_z : vs_x;
-    py3 *= hmul;
-    const float czz = cos_x * corr_z;
-    float cyy = vertical ? -sin_x * corr_z : corr_x;
-    cyy *= hmul;
-    const float top = pz * half + py3;
+    const StepProj sp = project(cur.db, cur.dn);
+    const float pz = sp.pz, py3 = sp.py3, czz = sp.czz, cyy = sp.cyy, top = sp.top;
     const uint32_t slen = ent.y & 0xffffu;
     g_u16* runs = slab + 2 + wofs;
 
@@ -1089,7 +1216,46 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
       }
     }
 
-    // ---- ordered replay of the steps that act
+    out.L = L;
+    out.mip = mip;
+    out.shift = shift;
+    out.slab = slab;
+    out.db = cur.db;
+    out.dn = cur.dn;
+    out.ent = ent;
+    out.F = F;
+    out.F2 = F2;
+    out.kF = kF;
+    out.ygF = ygF;
+    out.textureF = textureF;
+    out.s1F = s1F;
+    out.cand = cand;
+    out.drawF = drawF;
+    out.texF = texF;
+    out.s1rF = s1rF;
+    out.u1zF = u1zF;
+    out.u2dzF = u2dzF;
+    out.onez1F = onez1F;
+    out.onedz2F = onedz2F;
+    out.nel = nel;
+  };
+  // ---- ordered replay of the steps that act; false when the line has ended
+  auto replay = [&](const DdaPrepared& in, lds_u16* rc) -> bool {
+    const int L = in.L, mip = in.mip, shift = in.shift;
+    g_u16* slab = in.slab;
+    const uint2 ent = in.ent;
+    const bool valid = lane < L;
+    // Made again rather than held: the drawing wavefront of three gets db and
+    // dn, and the batch kernel has registers to spare that way (64 views 5.32
+    // -> 5.20 ms).
+    const StepProj sp = project(in.db, in.dn);
+    const float pz = sp.pz, py3 = sp.py3, czz = sp.czz, cyy = sp.cyy, top = sp.top;
+    const int F = in.F, F2 = in.F2, kF = in.kF, ygF = in.ygF, textureF = in.textureF;
+    const int s1F = in.s1F;
+    const bool cand = in.cand, drawF = in.drawF;
+    const float texF = in.texF, s1rF = in.s1rF, u1zF = in.u1zF, u2dzF = in.u2dzF;
+    const float onez1F = in.onez1F, onedz2F = in.onedz2F;
+    const uint32_t nel = in.nel;
     int cur_step = 0;
     bool done = false;
     for (;;) {
@@ -1431,13 +1597,20 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
     // ---- early end of the walk (WalkEnd): later steps lie beyond this
     // chunk's last crossing distance
     if (!done && L > 0 && !cnt.ended && wfloor < (float)ymin + (1.0f - WalkEnd::kAbs) &&
-        wend->done(readlane_f(cur.dn, L - 1), ymin, sc.mip[uni(mip)].top, sc.sy)) {
+        wend->done(readlane_f(in.dn, L - 1), ymin, sc.mip[uni(mip)].top, sc.sy)) {
       if (COUNT) cnt.end_walk();  // the counting variant walks on to count the reference's work
       else done = true;
     }
     return !done;
   };
-  if constexpr (!TWO) {
+  // a chunk prepared and replayed by one wavefront
+  auto chunk_step = [&](auto produce, const DdaChunk& cur, DdaChunk& nxt, bool& have_next) {
+    if (ymin >= ymax) return false;
+    DdaPrepared p;
+    prepare(produce, cur, nxt, have_next, rc, p);
+    return replay(p, rc);
+  };
+  if constexpr (WAVES == 1) {
     // the first step has no chunk of its own (L = 0) and only walks ahead
     DdaChunk cur, nxt;
     cur.L = 0;
@@ -1457,6 +1630,106 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
       cur.db = nxt.db;
       cur.dn = nxt.dn;
       cur.ent = nxt.ent;
+    }
+  } else if constexpr (WAVES == 3) {
+    LineRings& r = *rings;
+    if (producer && lane == 0) {
+      r.walked = r.prepared = r.taken = r.replayed = r.stop = 0;
+      r.walk_total = r.prep_total = INT32_MAX;
+      r.horizon = ymin;
+    }
+    __syncthreads();
+    if (producer) {
+      // chunk n is walked, then chunk n-1 (whose gather ran meanwhile)
+      // completed and chunk n's gather issued
+      uint2 ent = make_uint2(0u, 0u);
+      int s = 0, before = 0;  // slots of chunks n, n-1
+      for (int n = 0;; n++) {
+        int stop;
+        for (;;) {
+          const int taken = ring_read(r.taken);
+          stop = ring_read(r.stop);
+          ymin = ring_read(r.horizon);
+          if (stop || n - taken < kWalkSlots) break;
+          __builtin_amdgcn_s_sleep(8);
+        }
+        if (stop) break;
+        wave_sync();
+        DdaChunk c;
+        const bool more = dda_next_chunk<true>(wk, c, sc, *lc, zfar, ymin, dl, lane);
+        if (n > 0) {
+          r.ent[before][lane] = ent;  // waits for the gather
+          ring_write(r.walked, n, lane);
+        }
+        if (!more) {
+          ring_write(r.walk_total, n, lane);
+          break;
+        }
+        dda_gather(wk, c, vpx, vpz, fix_xf, fix_yf, lane);
+        ent = c.ent;
+        r.db[s][lane] = c.db;
+        r.dn[s][lane] = c.dn;
+        if (lane == 0) {
+          r.slab[s] = c.slab;
+          r.L[s] = c.L;
+          r.mip[s] = c.mip;
+          r.shift[s] = c.shift;
+        }
+        before = s;
+        s = s == kWalkSlots - 1 ? 0 : s + 1;
+      }
+    } else if (!drawer) {
+      const std::false_type no;
+      DdaChunk cur, unused;
+      bool hu = false;
+      int s = 0, n = 0;
+      for (;; n++) {
+        int stop, walked;
+        for (;;) {
+          walked = ring_read(r.walked);
+          const int total = ring_read(r.walk_total);
+          stop = ring_read(r.stop);
+          const int replayed = ring_read(r.replayed);
+          ymin = ring_read(r.horizon);
+          if (stop || total <= n || (walked > n && n - replayed < kPrepSlots)) break;
+          __builtin_amdgcn_s_sleep(4);
+        }
+        if (stop || walked <= n) break;
+        wave_sync();
+        cur.L = uni(r.L[s]);
+        cur.mip = uni(r.mip[s]);
+        cur.shift = uni(r.shift[s]);
+        cur.slab = (g_u16*)uni64((uint64_t)r.slab[s]);
+        cur.db = r.db[s][lane];
+        cur.dn = r.dn[s][lane];
+        cur.ent = r.ent[s][lane];
+        ring_write(r.taken, n + 1, lane);
+        DdaPrepared p;
+        prepare(no, cur, unused, hu, rc + (n & 1) * (64 * RC), p);
+        prep_put(r, n & 1, p, lane);
+        ring_write(r.prepared, n + 1, lane);
+        s = s == kWalkSlots - 1 ? 0 : s + 1;
+      }
+      ring_write(r.prep_total, n, lane);
+    } else {
+      for (int n = 0;; n++) {
+        int prepared;
+        for (;;) {
+          prepared = ring_read(r.prepared);
+          const int total = ring_read(r.prep_total);
+          if (prepared > n || total <= n) break;
+          __builtin_amdgcn_s_sleep(4);
+        }
+        if (prepared <= n) break;
+        wave_sync();
+        DdaPrepared p;
+        prep_get(r, n & 1, p, lane);
+        p.nel = 0;
+        if (!replay(p, rc + (n & 1) * (64 * RC))) break;
+        ring_write(r.horizon, ymin, lane);
+        ring_write(r.replayed, n + 1, lane);
+      }
+      ring_write(r.stop, 1, lane);
     }
   } else {
     // Round i: slot i%3 holds chunk i complete, slot (i+1)%3 chunk i+1's DDA
