@@ -186,7 +186,8 @@ typedef struct {
                               renders: the batched kernels keep one wavefront
                               per line, which uses a full GPU better) */
   int32_t persistent_waves; /* wavefronts per CU of the persistent batch kernel
-                               (0 = default 16, else 4..32) */
+                               (0 = default: 20, or 16 with lane-parallel
+                               element replay; else 4..32) */
   int32_t order;           /* 0 = view order, 1 = longest views first */
   int32_t run_cache;       /* LDS run-cache words per candidate column of the
                               wavefront-per-line kernels (24, 40 or 56; 0 =

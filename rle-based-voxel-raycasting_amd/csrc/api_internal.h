@@ -78,7 +78,13 @@ rlevox_status ctx_bind(rlevox_ctx* ctx);
 // the batch shape from the descriptor block, whose address never changes).
 struct BatchSlot {
   static constexpr int kMaxViews = 4096;
-  static constexpr int kWavesPerCU = 16;
+  // Wavefronts per CU of the persistent raycast, as many as its registers let
+  // reside: its registers are capped at 96 for it (64 mixed views / 40 served
+  // requests with 16 wavefronts of 128 registers 5.16 / 2.96 ms, 16 of 96
+  // 5.27 / 2.90, 20 of 96 4.87 / 2.79, 24 of 80 5.67 / 3.30; 16 small views,
+  // too few for either, 443 and 449 us).  With lane-parallel element replay
+  // 16 of 128: more would spill in the walk.
+  static constexpr int kWavesPerCU = 20, kWavesPerCUPar = 16;
   rlevox_ctx* ctx = nullptr;
   hipStream_t stream = nullptr;
   Scratch scratch, descs;
@@ -180,4 +186,9 @@ struct rlevox_scene {
   std::vector<void*> allocs;
   uint64_t bytes = 0;
   float mean_runs = 0;  // runs per level-0 column, from a sample taken at upload
+  // Lane-parallel element replay for columns of more than kParRuns runs on
+  // average (the generated 4096^2 terrains: 5.6-5.9; the 16384^2 terrain's
+  // settings give 7.6 already at 4096^2).
+  static constexpr float kParRuns = 7.0f;
+  bool par_elems() const { return mean_runs > kParRuns; }
 };

@@ -39,16 +39,15 @@ __device__ inline int find_view(const ViewDesc* __restrict__ v, int n, int64_t g
 
 // Persistent: each wavefront takes the next line of the batch until the
 // queue is drained; every wavefront reaches the exit test each iteration.
-// Register use is capped for four wavefronts per SIMD (16 per CU, the
-// default launch): two cold values spill, and the batch runs faster than
-// at the three wavefronts per SIMD its natural registers allow.  PAR: the replay prepares a column's elements across the lanes and
+// Register use is capped for five wavefronts per SIMD (BatchSlot::kWavesPerCU:
+// one value of a line's setup spills), four with PAR.  PAR: the replay prepares a column's elements across the lanes and
 // visits only those that can act, as the plain kernels do; it spills more
 // and pays only where columns hold many runs (served mix with three 16384^2
 // scenes resident: 4165 -> 4769 Mrays/s; 64 views over 4096^2 terrains:
 // 10.36 -> 10.86 ms), so a batch takes it by its scenes' runs per column
 // unless the tuning says otherwise.  RC: LDS run-cache words per column.
 template <bool PAR, int RC>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_raycast_batch(BatchHeader* __restrict__ h,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PAR ? 4 : 5))) void k_raycast_batch(BatchHeader* __restrict__ h,
                                                       const ViewDesc* __restrict__ views_) {
   __shared__ uint32_t bits[(RLEVOX_MAX_RS + 31) / 32];
   __shared__ uint4 rcache[64 * RC / 8];
@@ -247,16 +246,13 @@ rlevox_status BatchSlot::prepare(const rlevox_view* views, int n, const rlevox_r
   }
   std::vector<int> order(n);
   std::iota(order.begin(), order.end(), 0);
-  waves = tuning.persistent_waves ? tuning.persistent_waves : kWavesPerCU;
   if (tuning.order == 1)
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost[a] > cost[b]; });
-  // Lane-parallel element replay when some scene's columns hold more than
-  // kParRuns runs on average (the generated 4096^2 terrains: 5.6-5.9; the
-  // 16384^2 terrain's settings give 7.6 already at 4096^2).
-  constexpr float kParRuns = 7.0f;
-  par_elems = false;
-  for (int i = 0; i < n; i++) par_elems = par_elems || views[i].scene->mean_runs > kParRuns;
+  par_elems = false;  // some scene's columns call for it
+  for (int i = 0; i < n; i++) par_elems = par_elems || views[i].scene->par_elems();
   if (tuning.batch_par) par_elems = tuning.batch_par == 2;
+  waves = tuning.persistent_waves ? tuning.persistent_waves
+                                  : (par_elems ? kWavesPerCUPar : kWavesPerCU);
   // 24, 40: 64 mixed views 5.19, 5.21 ms, 16 small ones 446, 449 us
   run_cache = tuning.batch_run_cache ? tuning.batch_run_cache : 24;
   // scratch layout: per view ray buffer, line clip ranges, composed colour

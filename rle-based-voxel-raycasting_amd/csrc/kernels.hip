@@ -30,11 +30,13 @@ __global__ __launch_bounds__(256) void k_raycast_plain(SceneDev sc, rlevox_rayma
 // at the head of the launch.  Measured 1-6% faster than index order on
 // 1080p and 4K flythroughs and random views, equal on grazing views.
 //
-// One wavefront (= one block) per ray line.  Registers are capped for four
-// wavefronts per SIMD (4096 resident lines on 256 CUs); uncapped the
-// compiler takes 140 and only three fit.
-template <bool COUNT, int RC>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_raycast_wave(SceneDev sc, rlevox_raymap rm,
+// One wavefront (= one block) per ray line.  Registers are capped for five
+// wavefronts per SIMD (5120 resident lines on 256 CUs), four with the
+// lane-parallel element replay (PAR), whose walk would spill.  It pays where
+// columns hold many runs: four 4K frames over terrain of 5.9 runs a column
+// 926 us with it, 905 without; four grazing ones over 7.6 runs 820 and 850.
+template <bool COUNT, bool PAR, int RC>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PAR ? 4 : 5))) void k_raycast_wave(SceneDev sc, rlevox_raymap rm,
                                                      uint32_t* __restrict__ raybuf,
                                                      int32_t* __restrict__ clip,
                                                      unsigned long long* counts) {
@@ -44,7 +46,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
   extern __shared__ uint32_t lds[];
   if ((int)blockIdx.x >= rm.map_line_count) return;
   const int x = rm.map_line_count - 1 - (int)blockIdx.x;  // last line first
-  render_line_wave<COUNT, 1, true, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
+  render_line_wave<COUNT, 1, PAR, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
                                            clip + 2 * x, lds, dda,
                                            (lds_u16*)rcache, sweep, counts);
 }
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(256) void k_gapfill(int W, int H, const uint16_t* _
 
 template <int RC>
 static void launch_waves(const SceneDev& sc, const rlevox_raymap& rm, uint32_t* raybuf,
-                        int32_t* clip, int waves, hipStream_t s) {
+                         int32_t* clip, int waves, bool par, hipStream_t s) {
   const size_t lds = (size_t)bitmap_words(rm.rs) * sizeof(uint32_t);
   if (waves == 3)
     hipLaunchKernelGGL(k_raycast_wave3<RC>, dim3(rm.map_line_count), dim3(192), lds, s, sc, rm,
@@ -144,13 +146,16 @@ static void launch_waves(const SceneDev& sc, const rlevox_raymap& rm, uint32_t* 
   else if (waves == 2)
     hipLaunchKernelGGL(k_raycast_wave2<RC>, dim3(rm.map_line_count), dim3(128), lds, s, sc, rm,
                        raybuf, clip);
+  else if (par)
+    hipLaunchKernelGGL((k_raycast_wave<false, true, RC>), dim3(rm.map_line_count), dim3(64), lds, s,
+                       sc, rm, raybuf, clip, nullptr);
   else
-    hipLaunchKernelGGL((k_raycast_wave<false, RC>), dim3(rm.map_line_count), dim3(64), lds, s, sc,
-                       rm, raybuf, clip, nullptr);
+    hipLaunchKernelGGL((k_raycast_wave<false, false, RC>), dim3(rm.map_line_count), dim3(64), lds, s,
+                       sc, rm, raybuf, clip, nullptr);
 }
 
 hipError_t launch_raycast_plain(const SceneDev& sc, const rlevox_raymap& rm, uint32_t* raybuf,
-                                int32_t* clip, int block, int run_cache, hipStream_t s,
+                                int32_t* clip, int block, int run_cache, bool par, hipStream_t s,
                                 unsigned long long* counts) {
   const int lines = rm.map_line_count;
   if (lines <= 0) return hipSuccess;
@@ -162,14 +167,14 @@ hipError_t launch_raycast_plain(const SceneDev& sc, const rlevox_raymap& rm, uin
     if (run_cache == 0) run_cache = 24;
     if (counts) {  // counting walks with one wavefront and the default run cache
       const size_t lds = (size_t)bitmap_words(rm.rs) * sizeof(uint32_t);
-      hipLaunchKernelGGL((k_raycast_wave<true, kRunCache>), dim3(lines), dim3(64), lds, s, sc, rm,
+      hipLaunchKernelGGL((k_raycast_wave<true, true, kRunCache>), dim3(lines), dim3(64), lds, s, sc, rm,
                          raybuf, clip, counts);
     } else if (run_cache == 24) {
-      launch_waves<24>(sc, rm, raybuf, clip, block, s);
+      launch_waves<24>(sc, rm, raybuf, clip, block, par, s);
     } else if (run_cache == 56) {
-      launch_waves<56>(sc, rm, raybuf, clip, block, s);
+      launch_waves<56>(sc, rm, raybuf, clip, block, par, s);
     } else {
-      launch_waves<kRunCache>(sc, rm, raybuf, clip, block, s);
+      launch_waves<kRunCache>(sc, rm, raybuf, clip, block, par, s);
     }
     return hipGetLastError();
   }

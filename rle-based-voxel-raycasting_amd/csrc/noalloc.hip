@@ -86,7 +86,8 @@ extern "C" rlevox_status rlevox_render_noalloc(rlevox_ctx* ctx, const rlevox_sce
   }
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = launch_raycast_plain(scene->dev, rm, raybuf, clip,
-                                      ctx->tuning_block(t, rm.map_line_count, rm.rs), t.run_cache, s);
+                                      ctx->tuning_block(t, rm.map_line_count, rm.rs), t.run_cache,
+                                      scene->par_elems(), s);
   if (e != hipSuccess) return hip_fail(e, "render_noalloc: raycast launch");
   e = launch_compose(rm, raybuf, clip, cmp, d_depth, s);
   if (e != hipSuccess) return hip_fail(e, "render_noalloc: compose launch");

@@ -669,13 +669,12 @@ __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const Scene& sc,
 }
 
 // Cell of each step of the chunk just walked (Cuda_Render.h:416-442) and the
-// load of its pointer-map entry (left in flight).
+// load of its pointer-map entry (left in flight).  fix_x, fix_z: what the fix-up
+// adds to the cell of an x, a z crossing (0 or -1).
 __device__ inline void dda_gather(const DdaWalk& w, DdaChunk& c, float vpx, float vpz,
-                                  float fix_xf, float fix_yf, int lane) {
-  const int fix_x = (int)((float)(1 - c.ib) * fix_xf);
-  const int fix_z = (int)((float)c.ib * fix_yf);
-  const int voxel_x = d_f2i(vpx + c.pbx) + fix_x;
-  const int voxel_z = d_f2i(vpz + c.pby) + fix_z;
+                                  int fix_x, int fix_z, int lane) {
+  const int voxel_x = d_f2i(vpx + c.pbx) + (c.ib ? 0 : fix_x);
+  const int voxel_z = d_f2i(vpz + c.pby) + (c.ib ? fix_z : 0);
   const int vx = (voxel_x >> w.mip) & (w.gridx - 1);
   const int vz = (voxel_z >> w.mip) & (w.gridz - 1);
   c.ent = make_uint2(0u, 0u);
@@ -960,19 +959,18 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
   const float vpx = uni_f(rm.position[0]), vpy = uni_f(rm.position[1]), vpz = uni_f(rm.position[2]);
   const float ddx = ray_x * rm.cos_y + ray_z * rm.sin_y;
   const float ddy = ray_x * rm.sin_y - ray_z * rm.cos_y;
-  float fix_xf = -1, fix_yf = -1, sign_x = -1, sign_y = -1;
+  float sign_x = -1, sign_y = -1;
   float frac_x = vpx - (float)uni(d_f2i(vpx));
   float frac_y = vpz - (float)uni(d_f2i(vpz));
   if (ddx >= 0) {
-    fix_xf = 0;
     sign_x = 1;
     frac_x = 1 - frac_x;
   }
   if (ddy >= 0) {
-    fix_yf = 0;
     sign_y = 1;
     frac_y = 1 - frac_y;
   }
+  const int fix_x = uni(ddx >= 0 ? 0 : -1), fix_z = uni(ddy >= 0 ? 0 : -1);
   DdaWalk wk;
   {
     const float g0y = ddy / fabsf(ddx), g1x = ddx / fabsf(ddy);
@@ -1189,7 +1187,7 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
     __builtin_amdgcn_s_waitcnt(kWaitLoads);
     // ---- next chunk's pointer gather: in flight during this chunk's replay
     if constexpr (decltype(produce)::value) {
-      if (have_next) dda_gather(wk, nxt, vpx, vpz, fix_xf, fix_yf, lane);
+      if (have_next) dda_gather(wk, nxt, vpx, vpz, fix_x, fix_z, lane);
     }
     wave_sync();  // run cache filled
     if (cand) {  // F2: projected top of the next element the loop tests
@@ -1665,7 +1663,7 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
           ring_write(r.walk_total, n, lane);
           break;
         }
-        dda_gather(wk, c, vpx, vpz, fix_xf, fix_yf, lane);
+        dda_gather(wk, c, vpx, vpz, fix_x, fix_z, lane);
         ent = c.ent;
         r.db[s][lane] = c.db;
         r.dn[s][lane] = c.dn;
@@ -1752,7 +1750,7 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
         ring_put_dda(r, s, p, more, lane);
         if (pend) r.ent[s1][lane] = ent;  // waits for the gather
         if (more) {
-          dda_gather(wk, p, vpx, vpz, fix_xf, fix_yf, lane);
+          dda_gather(wk, p, vpx, vpz, fix_x, fix_z, lane);
           ent = p.ent;
         }
         pend = more;
