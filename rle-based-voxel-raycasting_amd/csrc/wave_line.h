@@ -670,11 +670,12 @@ __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const Scene& sc,
 
 // Cell of each step of the chunk just walked (Cuda_Render.h:416-442) and the
 // load of its pointer-map entry (left in flight).  fix_x, fix_z: what the fix-up
-// adds to the cell of an x, a z crossing (0 or -1).
+// adds to the cell of an x, a z crossing (0 or -1; as floats: integer selects
+// made 320x240 2%, 1280x720 1% slower).
 __device__ inline void dda_gather(const DdaWalk& w, DdaChunk& c, float vpx, float vpz,
-                                  int fix_x, int fix_z, int lane) {
-  const int voxel_x = d_f2i(vpx + c.pbx) + (c.ib ? 0 : fix_x);
-  const int voxel_z = d_f2i(vpz + c.pby) + (c.ib ? fix_z : 0);
+                                  float fix_x, float fix_z, int lane) {
+  const int voxel_x = d_f2i(vpx + c.pbx) + (int)((float)(1 - c.ib) * fix_x);
+  const int voxel_z = d_f2i(vpz + c.pby) + (int)((float)c.ib * fix_z);
   const int vx = (voxel_x >> w.mip) & (w.gridx - 1);
   const int vz = (voxel_z >> w.mip) & (w.gridz - 1);
   c.ent = make_uint2(0u, 0u);
@@ -970,7 +971,7 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
     sign_y = 1;
     frac_y = 1 - frac_y;
   }
-  const int fix_x = uni(ddx >= 0 ? 0 : -1), fix_z = uni(ddy >= 0 ? 0 : -1);
+  const float fix_x = uni_f(ddx >= 0 ? 0.0f : -1.0f), fix_z = uni_f(ddy >= 0 ? 0.0f : -1.0f);
   DdaWalk wk;
   {
     const float g0y = ddy / fabsf(ddx), g1x = ddx / fabsf(ddy);
