@@ -137,9 +137,10 @@ typedef struct {
   uint64_t spans;       /* spans drawn */
   uint64_t col_loads;   /* colours read = texels drawn (2 B) */
   uint64_t cleared;     /* texels cleared (4 B) */
-  /* The same for the walk as the kernels make it: a line's walk ends as soon
-   * as no later step can draw (the fields above count the reference's walk
-   * to the far distance; spans, colours and cleared texels are equal). */
+  /* The same for the walk up to where the kernels end it: as soon as no later
+   * step can draw (the fields above count the reference's walk to the far
+   * distance; spans, colours and cleared texels are equal).  The kernels also
+   * step over stretches on the way that cannot draw; these count here. */
   uint64_t walk_steps;
   uint64_t walk_ptr_loads;
   uint64_t walk_rle_loads;
@@ -177,9 +178,9 @@ typedef struct {
                               consecutive DDA steps); 16, 32 or 64 = one lane
                               per line */
   int32_t waves_per_block; /* 1..4; with lines_per_wave 1: 1 = one wavefront
-                              both walks and draws a line, 2 or 4 = two
+                              both walks and draws a line, 2 or 3 = two
                               wavefronts per line, one walking the DDA ahead
-                              of the one drawing, 3 = three, with one between
+                              of the one drawing, 4 = three, with one between
                               them that projects and fetches columns, 0 = by
                               the frame: one when it is wider than 2560,
                               three up to 1792 lines, else two (single

@@ -139,12 +139,9 @@ struct rlevox_ctx {
   }
   // Widest ray-buffer line (screen width) up to which the automatic choice
   // walks each line with several wavefronts, one on the DDA and one drawing.
-  // Measured over the 100-pose flythrough of the 4096^2 terrain (mean
-  // raycast ms, two wavefronts / one with a 56-word run cache): 640x480
-  // 0.091 / 0.122, 1280x720 0.100 / 0.128, 1920x1080 0.118 / 0.141,
-  // 2048x1152 0.124 / 0.147, 2560x1440 0.142 / 0.160 (two better at every
-  // line count, up to 4096 and more lines), 3200x1800 0.210 / 0.186,
-  // 3840x2160 0.251 / 0.229.
+  // Whole frames over a flythrough of the 4096^2 terrain, us with two
+  // wavefronts / one: 1920x1080 133 / 150, 2560x1440 161 / 170, 3200x1800
+  // 221 / 198, 3840x2160 252 / 225.
   static constexpr int kTwoWaveMaxWidth = 2560;
   // Lines up to which a line of that width is walked by three wavefronts: the
   // lines whose LDS (21 KB each) the 256 compute units hold at once.  With
@@ -161,7 +158,7 @@ struct rlevox_ctx {
     if (t.lines_per_wave == 1) {
       if (t.waves_per_block == 0)
         return rs > kTwoWaveMaxWidth ? 1 : lines > kThreeWaveMaxLines ? 2 : 3;
-      return t.waves_per_block == 4 ? 2 : t.waves_per_block;
+      return t.waves_per_block == 4 ? 3 : t.waves_per_block == 1 ? 1 : 2;
     }
     int block = t.lines_per_wave * t.waves_per_block;
     const size_t lane_bytes = (size_t)rlevox::bitmap_words(rs) * sizeof(uint32_t);

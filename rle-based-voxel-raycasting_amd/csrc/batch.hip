@@ -40,9 +40,9 @@ __device__ inline int find_view(const ViewDesc* __restrict__ v, int n, int64_t g
 // Persistent: each wavefront takes the next line of the batch until the
 // queue is drained; every wavefront reaches the exit test each iteration.
 // Register use is capped for five wavefronts per SIMD (BatchSlot::kWavesPerCU:
-// one value of a line's setup spills), four with PAR.  PAR: the replay prepares a column's elements across the lanes and
-// visits only those that can act, as the plain kernels do; it spills more
-// and pays only where columns hold many runs (served mix with three 16384^2
+// one value of a line's setup spills), four with PAR.  PAR: the replay
+// prepares a column's elements across the lanes and visits only those that
+// can act; it takes more registers and pays only where columns hold many runs (served mix with three 16384^2
 // scenes resident: 4165 -> 4769 Mrays/s; 64 views over 4096^2 terrains:
 // 10.36 -> 10.86 ms), so a batch takes it by its scenes' runs per column
 // unless the tuning says otherwise.  RC: LDS run-cache words per column.

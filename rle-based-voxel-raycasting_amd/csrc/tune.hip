@@ -18,7 +18,7 @@ namespace {
 // lane per line in blocks of 16..256 lanes.
 const rlevox_tuning kCandidates[] = {
     {1, 1, 0, 1, 40}, {1, 2, 0, 1, 40}, {1, 1, 0, 1, 24}, {1, 2, 0, 1, 24}, {1, 1, 0, 1, 56},
-    {1, 2, 0, 1, 56}, {1, 3, 0, 1, 24}, {1, 3, 0, 1, 40}, {64, 1, 0, 1},    {64, 2, 0, 1},    {64, 4, 0, 1},    {32, 1, 0, 1},
+    {1, 2, 0, 1, 56}, {1, 4, 0, 1, 24}, {1, 4, 0, 1, 40}, {64, 1, 0, 1},    {64, 2, 0, 1},    {64, 4, 0, 1},    {32, 1, 0, 1},
     {32, 2, 0, 1},    {16, 1, 0, 1},    {16, 4, 0, 1},
 };
 
@@ -157,7 +157,7 @@ extern "C" rlevox_status rlevox_autotune_batch(rlevox_ctx* ctx, const rlevox_vie
   if (e != hipSuccess) st = hip_fail(e, "autotune_batch setup");
   // the batch shape: persistent wavefronts per CU, view order, run-cache
   // depth and element replay, all combinations
-  const int kWaves[] = {8, 12, 16, 20, 24}, kOrder[] = {0, 1}, kRc[] = {24, 40, 56}, kPar[] = {1, 2};
+  const int kWaves[] = {8, 12, 16, 24}, kOrder[] = {0, 1}, kRc[] = {24, 40, 56}, kPar[] = {1, 2};
   rlevox_tuning win = saved;
   double win_ms = 0;
   bool have = false;

@@ -3,9 +3,9 @@
 //
 //  1. DDA chunk: up to 64 DDA steps per pass, lane k taking step k.  The
 //     crossing distances and positions are repeated fp32 additions
-//     (Cuda_Render.h:398-414) of six independent sequences; their terms
-//     0..63 are computed side by side with the same additions the walk
-//     makes, and the x/z order is the merge order of the two distance
+//     (Cuda_Render.h:398-414) of six independent sequences, whose terms
+//     the lanes take from a closed form (dda_terms.h) that gives the same
+//     values; the x/z order is the merge order of the two distance
 //     sequences (ties go to x: the walk takes z only when strictly closer).
 //  2. Gather: each lane loads its cell's pointer-map entry, one round trip
 //     for the whole chunk, issued one chunk ahead (software pipeline).
@@ -526,7 +526,8 @@ __device__ inline void dda_chain(DdaWalk& w, DdaChunk& c, int L, float* dl, int 
   wave_sync();
 }
 
-// What the walk's own constants cost to hold across a line goes to LDS.
+// The line's constants, held in LDS: in registers across the walk they cost
+// wavefronts.
 struct LineConsts {
   WalkEnd end;
   SkipLine line;

@@ -49,7 +49,7 @@ def test_three_waves(ctx, oracle, c1_scene, dev, view, depth, size):
     alt, pitch, yaw, mip, far = VIEWS[view]
     row = workloads.surface_row(c1_scene.mips[0], 300.0, 200.0)
     pose = workloads.pose(300.0, alt - row, 200.0, pitch, yaw)
-    check(ctx, oracle, dev, c1_scene.mips, pose, size[0], size[1], mip, far, waves_per_block=3,
+    check(ctx, oracle, dev, c1_scene.mips, pose, size[0], size[1], mip, far, waves_per_block=4,
           run_cache=depth)
 
 
