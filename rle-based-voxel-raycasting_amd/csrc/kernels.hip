@@ -35,6 +35,8 @@ __global__ __launch_bounds__(256) void k_raycast_plain(SceneDev sc, rlevox_rayma
 // lane-parallel element replay (PAR), whose walk would spill.  It pays where
 // columns hold many runs: four 4K frames over terrain of 5.9 runs a column
 // 926 us with it, 905 without; four grazing ones over 7.6 runs 820 and 850.
+// Without it the walk's constants stay in registers (read again, a product of
+// each chunk's projection spills: 976 against 963 us).
 template <bool COUNT, bool PAR, int RC>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PAR ? 4 : 5))) void k_raycast_wave(SceneDev sc, rlevox_raymap rm,
                                                      uint32_t* __restrict__ raybuf,
@@ -46,7 +48,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PAR ? 4 : 5)
   extern __shared__ uint32_t lds[];
   if ((int)blockIdx.x >= rm.map_line_count) return;
   const int x = rm.map_line_count - 1 - (int)blockIdx.x;  // last line first
-  render_line_wave<COUNT, 1, PAR, RC>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
+  render_line_wave<COUNT, 1, PAR, RC, !PAR>(x, sc, rm, raybuf + (size_t)x * (size_t)rm.rs,
                                            clip + 2 * x, lds, dda,
                                            (lds_u16*)rcache, sweep, counts);
 }

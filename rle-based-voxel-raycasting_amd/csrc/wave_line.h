@@ -535,14 +535,19 @@ struct LineConsts {
 constexpr int kLineConstWords = (int)(sizeof(LineConsts) / 4);
 
 // The bounds of the window that begins `ahead` steps on, n steps before the
-// next mip switch or the far distance.
-template <class Scene>
+// next mip switch or the far distance.  HOLD: the line's constants may stay in
+// registers around the calls; else each call reads them again (held, the batch
+// kernel spills 16 bytes: 64 views 5.07 against 4.97 ms).
+template <bool HOLD, class Scene>
 __device__ inline void dda_look_ahead(DdaWalk& w, const Scene& sc, const LineConsts& lc,
                                       int ahead, int n, int lane) {
+  if (!HOLD) asm volatile("" ::: "memory");
   const float sA = readlane_f(w.q.s, 0), sB = readlane_f(w.q.s, 1);
   const float gA = readlane_f(w.g, 0), gB = readlane_f(w.g, 1);
-  const float r = __builtin_amdgcn_rcpf(gA + gB);
-  const SkipBase b{w.px, w.py, w.dnow, sA, sB, gA, gB, (sB - sA + gA) * r, gB * r};
+  const int other = w.idx ? 2 : 4;  // the sequences of the other kind's positions
+  const SkipBase b = SkipBase::of(lc.line, w.px, w.py, w.dnow, sA, sB, gA, gB, w.idx ? sA : sB,
+                                  readlane_f(w.q.s, other), readlane_f(w.q.s, other + 1),
+                                  __builtin_amdgcn_rcpf(gA + gB));
   const SkipLevel v{w.mip, w.gridx, w.gridz, (skip_tops*)sc.mip[uni(w.mip)].tops, sc.mip[uni(w.mip)].top};
   const int t0 = ahead + lane * kSkipSteps;
   const float bound = skip_bound(lc.end, lc.line, b, v, sc.sy, t0, t0 + kSkipSteps);
@@ -557,9 +562,9 @@ constexpr int kSkipReach = 2048;
 
 // Advances the walk by one chunk of up to 64 steps.  SKIP: steps that cannot
 // draw above the horizon row ymin (a row the line has reached or passed) are
-// stepped over on the way.  Returns false when the line has reached the far
-// distance.
-template <bool SKIP, class Scene>
+// stepped over on the way.  HOLD: see dda_look_ahead.  Returns false when the
+// line has reached the far distance.
+template <bool SKIP, bool HOLD, class Scene>
 __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const Scene& sc,
                                       const LineConsts& lc, int zfar, int ymin, float* dl,
                                       int lane) {
@@ -596,7 +601,7 @@ __device__ inline bool dda_next_chunk(DdaWalk& w, DdaChunk& c, const Scene& sc,
     if (SKIP) {
       bool look = w.ofs >= w.end;
       for (;;) {
-        if (look) dda_look_ahead(w, sc, lc, hidden, n, lane);
+        if (look) dda_look_ahead<HOLD>(w, sc, lc, hidden, n, lane);
         const int at = max(w.ofs, 0) / kSkipSteps;  // the group of the next step
         const uint64_t vis = uni64(ballot(!skip_hidden(w.bound, ymin))) >> at;
         if (vis) {
@@ -844,13 +849,14 @@ __device__ inline void prep_get(const LineRings& r, int s, DdaPrepared& p, int l
 // precomputes a column's remaining elements across the lanes (pays where
 // steps often show several elements, as in grazing views of caved terrain;
 // the persistent batch kernel leaves it off, where its registers spill).
+// HOLD: see dda_look_ahead.
 // LDS arguments (rc holds kPrepSlots caches for three wavefronts): bits = the line's bitmap, dl = DDA scratch, rc = run cache,
 // sweep_lds = 64 ints for the horizon sweep followed by kLineConstWords words
 // for the line's constants.
 // Scene, Map: SceneDev and rlevox_raymap as kernel arguments or in constant
 // memory.
-template <bool COUNT, int WAVES = 1, bool PAR_ELEMS = true, int RC = kRunCache, class Scene,
-          class Map>
+template <bool COUNT, int WAVES = 1, bool PAR_ELEMS = true, int RC = kRunCache, bool HOLD = false,
+          class Scene, class Map>
 __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
                                         uint32_t* __restrict__ row_, int32_t* __restrict__ clip_,
                                         uint32_t* bits, float* dl, lds_u16* rc, int* sweep_lds,
@@ -1112,7 +1118,7 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
     constexpr int kWords = RC / 8;
     // ---- next chunk's DDA, before the cache's loads go out: an LDS access
     // waits for every load that writes LDS
-    if constexpr (decltype(produce)::value) have_next = dda_next_chunk<!COUNT>(wk, nxt, sc, *lc, zfar, ymin, dl, lane);
+    if constexpr (decltype(produce)::value) have_next = dda_next_chunk<!COUNT, HOLD>(wk, nxt, sc, *lc, zfar, ymin, dl, lane);
 
     // A wait for this wavefront's LDS reads (the last chunk's, of the cache)
     // before the loads may write it, and for the loads before it is read.
@@ -1656,7 +1662,7 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
         if (stop) break;
         wave_sync();
         DdaChunk c;
-        const bool more = dda_next_chunk<true>(wk, c, sc, *lc, zfar, ymin, dl, lane);
+        const bool more = dda_next_chunk<true, HOLD>(wk, c, sc, *lc, zfar, ymin, dl, lane);
         if (n > 0) {
           r.ent[before][lane] = ent;  // waits for the gather
           ring_write(r.walked, n, lane);
@@ -1748,7 +1754,7 @@ __device__ inline void render_line_wave(int x, const Scene& sc, const Map& rm,
       int s = 0, s1 = 2, s2 = 1;  // slots of chunks n, n-1, n-2
       for (int n = 0;; n++) {
         if (n >= 2 && !uni(r.have[s2])) break;
-        more = more && dda_next_chunk<true>(wk, p, sc, *lc, zfar, ymin, dl, lane);
+        more = more && dda_next_chunk<true, HOLD>(wk, p, sc, *lc, zfar, ymin, dl, lane);
         ring_put_dda(r, s, p, more, lane);
         if (pend) r.ent[s1][lane] = ent;  // waits for the gather
         if (more) {
