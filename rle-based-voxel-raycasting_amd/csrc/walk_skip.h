@@ -80,11 +80,24 @@ struct SkipBase {  // the last step taken, and what follows it
     return SkipBase{px, pz, dnow, sA, sB, gA, gB, (sB - sA + gA) * r, gB * r,
                     fmaf(-l.dirx, od, nx), fmaf(-l.dirz, od, nz)};
   }
-  // Distance of the t-th step from here (t = 0: of the base).
-  RLEVOX_HD float dist(float t) const {
-    const float i = fminf(fmaxf(floorf(e0 + e1 * t), 0.0f), t), j = t - i;
-    const float a = i > 0.0f ? sA + (i - 1.0f) * gA : dnow;
-    const float b = j > 0.0f ? sB + (j - 1.0f) * gB : dnow;
+  // Bounds of the distance of the t-th step from here (t = 0: of the base).
+  // They hold for any split t = i + j, as the guess may be off: for rays near
+  // an axis e1*t rounds by more than the share of the rarer crossings.  The
+  // t-th crossing is not beyond both x's i-th and z's j-th.  Either i of the
+  // first t are x's, and it is not before x's i-th, or j + 1 are z's, and it is
+  // not before z's j+1-st; likewise with x and z exchanged.
+  RLEVOX_HD float split(float t) const { return fminf(fmaxf(floorf(fmaf(e1, t, e0)), 0.0f), t); }
+  RLEVOX_HD float far_(float t) const {
+    const float i = split(t), j = t - i;
+    return fmaxf(fmaxf(fmaf(i - 1.0f, gA, sA), fmaf(j - 1.0f, gB, sB)), dnow);
+  }
+  RLEVOX_HD float near_(float t) const {
+    // a kind's 0-th crossing is at or before the base: a spacing before its
+    // next one, less the rounding of that sum
+    constexpr float kBelow = 0.99999988f;
+    const float i = split(t), j = t - i;
+    const float a = fminf(fmaf(i - 1.0f, gA, sA * kBelow), fmaf(j, gB, sB));
+    const float b = fminf(fmaf(j - 1.0f, gB, sB * kBelow), fmaf(i, gA, sA));
     return fmaxf(fmaxf(a, b), dnow);
   }
 };
@@ -124,8 +137,9 @@ RLEVOX_HD inline SkipRange skip_range(const SkipLine& l, const SkipBase& b, int 
   SkipRange r;
   // a step uses the distances and the position of its ends: steps t0..t1-1
   // those of t0..t1
-  const float lo0 = b.dist((float)t0), hi0 = b.dist((float)t1);
-  const float drift = (2e-6f + 1.2e-7f * (float)t1) * hi0;
+  const float f0 = (float)t0, f1 = f0 + (float)(t1 - t0);
+  const float lo0 = b.near_(f0), hi0 = b.far_(f1);
+  const float drift = fmaf(1.2e-7f, f1, 2e-6f) * hi0;
   r.lo = fmaxf(lo0 - drift, 0.0f);
   r.hi = hi0 + drift;
   // the two lines at distance 0; drift also holds what the positions' sums

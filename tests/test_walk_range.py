@@ -29,8 +29,8 @@ def _run(exe, *args):
     return r.stdout
 
 
-def _range(tmp_path, plant, mip):
-    out = _run(_build(tmp_path, "walk_range_check", ["WALK_RANGE_PLANT=%d" % plant]), mip, 20000000)
+def _range(tmp_path, plant, mip, steps=20000000):
+    out = _run(_build(tmp_path, "walk_range_check", ["WALK_RANGE_PLANT=%d" % plant]), mip, steps)
     m = re.search(r"groups (\d+), of two blocks a side (\d+), below lo (\d+), above hi (\d+), "
                   r"outside (\d+)", out)
     assert m, out
@@ -49,6 +49,13 @@ def test_every_step_is_in_its_groups_blocks(tmp_path, mip):
 @pytest.mark.parametrize("mip", [16384, 65536])
 def test_range_check_catches_a_missing_offset(tmp_path, mip):
     assert _range(tmp_path, 1, mip)["outside"] > 0
+
+
+@pytest.mark.parametrize("mip", [30, 1024, 4096])
+def test_no_step_is_nearer_than_its_group(tmp_path, mip):
+    """Near an axis too, where the guessed split of a group's steps between
+    the two kinds of crossing is off."""
+    assert _range(tmp_path, 0, mip, 100000000)["below"] == 0
 
 
 def _reach(exe, scene, mip):
