@@ -181,11 +181,12 @@ typedef struct {
                               both walks and draws a line, 2 or 3 = two
                               wavefronts per line, one walking the DDA ahead
                               of the one drawing, 4 = three, with one between
-                              them that projects and fetches columns, 0 = by
-                              the frame: one when it is wider than 2560,
-                              three up to 1792 lines, else two (single
-                              renders: the batched kernels keep one wavefront
-                              per line, which uses a full GPU better) */
+                              them that projects and fetches columns, where
+                              they are faster (frames at most 2560 wide of at
+                              most 1792 lines), else two, 0 = as 4, but one
+                              in frames wider than 2560 (single renders: the
+                              batched kernels keep one wavefront per line,
+                              which uses a full GPU better) */
   int32_t persistent_waves; /* wavefronts per CU of the persistent batch kernel
                                (0 = default: 20, or 16 with lane-parallel
                                element replay; else 4..32) */

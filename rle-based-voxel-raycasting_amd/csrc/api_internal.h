@@ -10,6 +10,7 @@
 
 #include "device.h"
 #include "internal.h"
+#include "line_waves.h"
 
 namespace rlevox {
 
@@ -137,29 +138,11 @@ struct rlevox_ctx {
     auto it = tuned.find(TuneKey{s, W, H});
     return it == tuned.end() ? tuning : it->second;
   }
-  // Widest ray-buffer line (screen width) up to which the automatic choice
-  // walks each line with several wavefronts, one on the DDA and one drawing.
-  // Whole frames over a flythrough of the 4096^2 terrain, us with two
-  // wavefronts / one: 1920x1080 133 / 150, 2560x1440 161 / 170, 3200x1800
-  // 221 / 198, 3840x2160 252 / 225.
-  static constexpr int kTwoWaveMaxWidth = 2560;
-  // Lines up to which a line of that width is walked by three wavefronts: the
-  // lines whose LDS (21 KB each) the 256 compute units hold at once.  With
-  // them all resident a frame takes as long as its longest line, which three
-  // wavefronts walk faster; beyond, lines wait for LDS (us per frame, three
-  // / two: 320x240, 441 lines, 83 / 91; 640x480, 882-1125 lines, 79 / 88;
-  // 1366x768, 1532-1654 lines, 98 / 99; 1280x720, 1626-1891 lines, 88 / 94;
-  // 1920x1080, 2048-3050 lines, 170 / 132).
-  static constexpr int kThreeWaveMaxLines = 1792;
   // 1 selects the wavefront-per-line kernel, 2 and 3 its forms with more;
   // otherwise lanes per block (16 or more), halved until the block's
   // per-lane bitmaps (ceil(rs/32) words each) fit the workgroup's LDS.
   int tuning_block(const rlevox_tuning& t, int lines, int rs) const {
-    if (t.lines_per_wave == 1) {
-      if (t.waves_per_block == 0)
-        return rs > kTwoWaveMaxWidth ? 1 : lines > kThreeWaveMaxLines ? 2 : 3;
-      return t.waves_per_block == 4 ? 3 : t.waves_per_block == 1 ? 1 : 2;
-    }
+    if (t.lines_per_wave == 1) return rlevox::line_waves(t.waves_per_block, lines, rs);
     int block = t.lines_per_wave * t.waves_per_block;
     const size_t lane_bytes = (size_t)rlevox::bitmap_words(rs) * sizeof(uint32_t);
     while (block > 16 && (size_t)block * lane_bytes > max_lds) block >>= 1;

@@ -13,7 +13,7 @@ using namespace rlevox;
 
 namespace {
 
-// Candidates: one, two or three wavefronts per line (lanes take consecutive DDA
+// Candidates: one, two or up to three wavefronts per line (lanes take consecutive DDA
 // steps) with an LDS run cache of 24, 40 or 56 words per column, and one
 // lane per line in blocks of 16..256 lanes.
 const rlevox_tuning kCandidates[] = {
