@@ -183,8 +183,9 @@ typedef struct {
                               of the one drawing, 4 = three, with one between
                               them that projects and fetches columns, where
                               they are faster (frames at most 2560 wide of at
-                              most 1792 lines), else two, 0 = as 4, but one
-                              in frames wider than 2560 (single renders: the
+                              most 1792 lines; 1536 or 1280 with a run cache
+                              of 40 or 56), else two, 0 = as 4, but one in
+                              frames wider than 2560 (single renders: the
                               batched kernels keep one wavefront per line,
                               which uses a full GPU better) */
   int32_t persistent_waves; /* wavefronts per CU of the persistent batch kernel

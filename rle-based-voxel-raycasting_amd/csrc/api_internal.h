@@ -10,6 +10,7 @@
 
 #include "device.h"
 #include "internal.h"
+#include "kernels.h"
 #include "line_waves.h"
 
 namespace rlevox {
@@ -116,7 +117,7 @@ hipError_t launch_copy_u128(void* dst, const void* src, uint64_t n16, hipStream_
 struct rlevox_ctx {
   int device = 0;
   int num_cus = 0;
-  size_t max_lds = 65536;  // LDS bytes one workgroup may take
+  size_t max_lds = 65536;  // LDS bytes one workgroup may take: a compute unit's
   char arch[64] = {0};
   std::mutex mu;  // guards the scratch buffers and tuning
   rlevox::Scratch raybuf, clip, ctmp, counts;
@@ -142,7 +143,10 @@ struct rlevox_ctx {
   // otherwise lanes per block (16 or more), halved until the block's
   // per-lane bitmaps (ceil(rs/32) words each) fit the workgroup's LDS.
   int tuning_block(const rlevox_tuning& t, int lines, int rs) const {
-    if (t.lines_per_wave == 1) return rlevox::line_waves(t.waves_per_block, lines, rs);
+    if (t.lines_per_wave == 1)
+      return rlevox::line_waves(
+          t.waves_per_block, lines, rs,
+          rlevox::three_wave_max_lines(num_cus, (int)max_lds, rlevox::raycast_wave3_lds(t.run_cache, rs)));
     int block = t.lines_per_wave * t.waves_per_block;
     const size_t lane_bytes = (size_t)rlevox::bitmap_words(rs) * sizeof(uint32_t);
     while (block > 16 && (size_t)block * lane_bytes > max_lds) block >>= 1;

@@ -7,13 +7,22 @@
 
 namespace rlevox {
 
+// Default run-cache depth of the wavefront kernels, in words.  With the cache
+// loaded straight into LDS the deeper ones save no time and hold LDS (us with
+// 24 / 40 / 56: four 1080p frames 572 / 574 / -, four at 4K 1120 / 1125 /
+// 1127, four grazing ones 969 / 971 / 976; 640x480 with three wavefronts 325 /
+// 327 / -).
+constexpr int kRunCacheDefault = 24;
+
 // block: 1, 2 or 3 = wavefronts per line, else lanes per block of the
 // lane-per-line kernel.  run_cache: LDS run-cache words of the wavefront
-// kernels (24, 40 or 56; 0 = 24; the counting variant always uses 40).  par:
+// kernels (24, 40 or 56; 0 = kRunCacheDefault; the counting variant always uses 40).  par:
 // lane-parallel element replay where one wavefront walks a line.
 hipError_t launch_raycast_plain(const SceneDev& sc, const rlevox_raymap& rm, uint32_t* raybuf,
                                 int32_t* clip, int block, int run_cache, bool par, hipStream_t s,
                                 unsigned long long* counts = nullptr);
+// LDS bytes of a line of the kernel with three wavefronts per line.
+int raycast_wave3_lds(int run_cache, int rs);
 hipError_t launch_compose(const rlevox_raymap& rm, const uint32_t* raybuf, const int32_t* clip,
                           uint16_t* col, int32_t* dep, hipStream_t s);
 // Smallest world row of a drawn run's top over the columns of each block of

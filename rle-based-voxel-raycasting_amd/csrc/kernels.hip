@@ -95,6 +95,12 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(5))) void k
                                           nullptr, &rings);
 }
 
+int raycast_wave3_lds(int run_cache, int rs) {
+  const int rc = run_cache ? run_cache : kRunCacheDefault;
+  return kPrepSlots * 64 * rc * 2 + (64 + kLineConstWords) * 4 + kDdaLds * 4 + (int)sizeof(LineRings) +
+         bitmap_words(rs) * 4;
+}
+
 // Tiles of 32x8 pixels, one pixel per thread: a tile's quotients and its loads
 // are one chain, hidden by other workgroups (64x16 tiles of four pixels per
 // thread: 640x480 5.0 against 4.9 us, 1366x768 7.4 against 6.5).
@@ -162,11 +168,7 @@ hipError_t launch_raycast_plain(const SceneDev& sc, const rlevox_raymap& rm, uin
   const int lines = rm.map_line_count;
   if (lines <= 0) return hipSuccess;
   if (block >= 1 && block <= 3) {  // wavefront kernels
-    // Default depth 24: with the cache loaded straight into LDS the deeper
-    // ones save no time and hold LDS (us with 24 / 40 / 56: four 1080p
-    // frames 572 / 574 / -, four at 4K 1120 / 1125 / 1127, four grazing ones
-    // 969 / 971 / 976; 640x480 with three wavefronts 325 / 327 / -).
-    if (run_cache == 0) run_cache = 24;
+    if (run_cache == 0) run_cache = kRunCacheDefault;
     if (counts) {  // counting walks with one wavefront and the default run cache
       const size_t lds = (size_t)bitmap_words(rm.rs) * sizeof(uint32_t);
       hipLaunchKernelGGL((k_raycast_wave<true, true, kRunCache>), dim3(lines), dim3(64), lds, s, sc, rm,

@@ -1,12 +1,13 @@
 // Prints the wavefronts per line (csrc/line_waves.h) for each line of input:
-// waves_per_block, lines, width.  Run by tests/test_line_waves.py.
+// waves_per_block, lines, width, LDS bytes of a line walked by three, on 256
+// compute units of 160 KB.  Run by tests/test_line_waves.py.
 #include <cstdio>
 
 #include "../../rle-based-voxel-raycasting_amd/csrc/line_waves.h"
 
 int main() {
-  int w, lines, rs;
-  while (std::scanf("%d %d %d", &w, &lines, &rs) == 3)
-    std::printf("%d\n", rlevox::line_waves(w, lines, rs));
+  int w, lines, rs, lds;
+  while (std::scanf("%d %d %d %d", &w, &lines, &rs, &lds) == 4)
+    std::printf("%d\n", rlevox::line_waves(w, lines, rs, rlevox::three_wave_max_lines(256, 163840, lds)));
   return 0;
 }

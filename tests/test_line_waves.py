@@ -31,4 +31,14 @@ def waves(tmp_path_factory):
     (4, 441, 320, 3), (4, 1792, 1366, 3), (4, 1793, 1366, 2), (4, 2048, 1920, 2),
     (4, 500, 2561, 2), (4, 9000, 3840, 2)])
 def test_waves_per_line(waves, setting, lines, width, want):
-    assert waves(setting, lines, width) == want
+    assert waves(setting, lines, width, 21040) == want
+
+
+# LDS of a line with a run cache of 24, 40 and 56 words, and at the edges of
+# the unit in which it is given out: seven, six, five lines a compute unit.
+@pytest.mark.parametrize("lds,most", [(21040, 1792), (25136, 1536), (29232, 1280), (23040, 1792),
+                                      (23041, 1536), (26880, 1536), (26881, 1280)])
+def test_three_waves_while_every_line_is_resident(waves, lds, most):
+    for setting in (0, 4):
+        assert waves(setting, most, 1366, lds) == 3
+        assert waves(setting, most + 1, 1366, lds) == 2
