@@ -157,9 +157,11 @@ rlevox_status rlevox_scene_upload(rlevox_ctx* ctx, const rlevox_mip* mips, int32
   void* dd = nullptr;
   size_t nblocks = 0;
   for (int i = 0; i < nmips; i++) nblocks += (size_t)skip_blocks(m[i].sx) * skip_blocks(m[i].sz);
-  hipError_t e = dev_malloc(&dd, sizeof(SceneDev) + sizeof(int32_t) * (RLEVOX_MAX_MIPS + nblocks));
+  const size_t dd_bytes = sizeof(SceneDev) + sizeof(int32_t) * (RLEVOX_MAX_MIPS + nblocks);
+  hipError_t e = dev_malloc(&dd, dd_bytes);
   if (e == hipSuccess) {
     s->allocs.push_back(dd);
+    s->bytes += dd_bytes;
     int32_t* d_top = (int32_t*)((char*)dd + sizeof(SceneDev));
     int32_t* d_blocks = d_top + RLEVOX_MAX_MIPS;
     e = launch_fill_u32((uint32_t*)d_top, (uint32_t)INT32_MAX, RLEVOX_MAX_MIPS, nullptr);
