@@ -97,8 +97,5 @@ struct WalkEnd {
     return ok && fmaxf(fmaxf(a, b), lim) < (float)ymin + (1.0f - kAbs);
   }
 };
-// 32-bit words of a WalkEnd kept in LDS by the wavefront kernels (read once
-// per chunk, so its values hold no registers across the walk).
-constexpr int kWalkEndWords = (int)(sizeof(WalkEnd) / 4);
 
 }  // namespace rlevox
