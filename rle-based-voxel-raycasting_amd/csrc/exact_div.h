@@ -4,11 +4,11 @@
 //
 // Markstein's theorems (IBM J. Res. Dev. 34, 1990): an estimate of 1/b within
 // one ulp, corrected once by its exact residual, is 1/b rounded to nearest
-// unless b's significand is all ones; and with that reciprocal an estimate
-// of a/b within one ulp, corrected once by its exact residual, is a/b rounded
-// to nearest.  The residuals are exact while nothing over- or underflows,
-// which the ranges of div_safe and
-// div_dividend_safe see to.
+// unless b's significand is all ones; and with that reciprocal a*r, corrected
+// once by its residual, is a/b rounded to nearest (one product and two fused
+// multiply-adds: Brisebarre, Muller, Raina, IEEE Trans. Comput. 53, 2004, who
+// start from this).  That holds while nothing over- or underflows, which the
+// ranges of div_safe and div_dividend_safe see to.
 #pragma once
 
 #include <math.h>

@@ -54,9 +54,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PAR ? 4 : 5)
 }
 
 // Two wavefronts (= one block) per ray line: wavefront 0 walks the DDA and
-// gathers the pointer map, wavefront 1 projects, caches and draws.  Capped at
-// six wavefronts per SIMD (80 registers; it takes 82 to 84 by itself, which
-// leaves five).
+// gathers the pointer map, wavefront 1 projects, caches and draws.  Six
+// wavefronts per SIMD (80 registers): it takes 77 as it is, 82 to 84 with the
+// line's constants held across the walk.
 template <int RC>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(6))) void k_raycast_wave2(SceneDev sc, rlevox_raymap rm,
                                                        uint32_t* __restrict__ raybuf,

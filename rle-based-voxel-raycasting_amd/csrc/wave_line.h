@@ -69,8 +69,9 @@ __device__ inline uint64_t uni64(uint64_t v) {
 __device__ inline bool lds_bit(const uint32_t* bits, int y) { return (bits[y >> 5] >> (y & 31)) & 1u; }
 
 // LDS hand-off between the lanes of one wavefront, on LDS that only this
-// wavefront uses (hand-offs between the two wavefronts of a line go through
-// the ring and its workgroup barrier).  A wavefront's LDS instructions
+// wavefront uses.  (Between the two wavefronts of a line ChunkRing and its
+// workgroup barrier hand over, between three LineRings and its counters, with
+// this point on either side of a counter.)  A wavefront's LDS instructions
 // execute in program order, so a write by one lane is seen by a later read
 // of another lane once the compiler keeps both on their side of this point.
 // Unlike a workgroup barrier, this emits no s_barrier and does not wait for
@@ -850,9 +851,9 @@ __device__ inline void prep_get(const LineRings& r, int s, DdaPrepared& p, int l
 // steps often show several elements, as in grazing views of caved terrain;
 // the persistent batch kernel leaves it off, where its registers spill).
 // HOLD: see dda_look_ahead.
-// LDS arguments (rc holds kPrepSlots caches for three wavefronts): bits = the line's bitmap, dl = DDA scratch, rc = run cache,
-// sweep_lds = 64 ints for the horizon sweep followed by kLineConstWords words
-// for the line's constants.
+// LDS arguments: bits = the line's bitmap, dl = DDA scratch, rc = run cache
+// (kPrepSlots of them for three wavefronts), sweep_lds = 64 ints for the
+// horizon sweep followed by kLineConstWords words for the line's constants.
 // Scene, Map: SceneDev and rlevox_raymap as kernel arguments or in constant
 // memory.
 template <bool COUNT, int WAVES = 1, bool PAR_ELEMS = true, int RC = kRunCache, bool HOLD = false,
